@@ -269,7 +269,8 @@ rccl_hip_status sort_buffer(rccl_hip_key_kind key, size_t value_bytes, rccl_hip_
 
 size_t merge_sort_lowering_bytes(size_t key_bytes_, size_t value_bytes, size_t n) {
   return align_up(n * key_bytes_, 256) + align_up(n * value_bytes, 256) +
-         layout(key_bytes_, value_bytes, n, true).total + plan_bytes();
+         layout(key_bytes_, value_bytes, n, true).total + plan_bytes() +
+         short_sample_bytes(key_bytes_, n);
 }
 
 // A stable LSD radix sort under the natural order or its reverse yields
@@ -318,7 +319,8 @@ rccl_hip_status merge_sort_lowering(rccl_hip_key_kind key, size_t value_bytes, b
                  (in_keys != out_keys || vals_copied ? PLAN_COPIES : 0u);
   return sort_buffer(key, value_bytes,
                      descending ? RCCL_HIP_ORDER_DESCENDING : RCCL_HIP_ORDER_ASCENDING, a,
-                     workspace_bytes - scratch - plan_bytes());
+                     workspace_bytes - scratch - plan_bytes() -
+                         short_sample_bytes(kb, n));
 }
 } // namespace radix
 } // namespace rccl_hip

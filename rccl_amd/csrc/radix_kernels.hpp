@@ -17,64 +17,11 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.hpp"
-#include "radix_plan.hpp"
+#include "radix_block_kernels.hpp"
+#include "radix_digits.hpp"
 
 namespace rccl_hip {
 namespace radix {
-
-struct NoValue {};
-
-enum class KeyClass { Unsigned, Signed, Float };
-
-// Order-preserving bit image of a key, with the float +-0 collapse applied
-// for digit extraction. Transforms: rccl-cub/src/ordering_backend/radix.rs:75-235
-// (unsigned identity, signed sign flip, float: negative -> all bits inverted,
-// otherwise sign flipped; descending = complement); collapse: :257-337 (the
-// ordered value 0x7f..f is read as 0x80..0, so -0.0 and +0.0 share every
-// digit). Stored keys are never rewritten.
-template <class Bits, KeyClass KC, bool DESC>
-struct KeyOps {
-  using SBits = typename std::make_signed<Bits>::type;
-  static constexpr int NBITS = int(sizeof(Bits) * 8);
-  static constexpr Bits SIGN = Bits(1) << (NBITS - 1);
-
-  // The order-preserving bijection, before the collapse. Onesweep passes keep
-  // keys in this form between passes: the first converts its raw input
-  // (image), the last its output back (raw), and every digit in between
-  // needs only the collapse (image_digit): about half the ALU work per digit
-  // for float keys.
-  __device__ static __forceinline__ Bits image(Bits raw) {
-    Bits x = raw;
-    if constexpr (KC == KeyClass::Signed) x ^= SIGN;
-    if constexpr (KC == KeyClass::Float)
-      x ^= static_cast<Bits>(static_cast<SBits>(raw) >> (NBITS - 1)) | SIGN;
-    if constexpr (DESC) x = ~x;
-    return x;
-  }
-  __device__ static __forceinline__ Bits raw(Bits x) {
-    if constexpr (DESC) x = ~x;
-    if constexpr (KC == KeyClass::Signed) x ^= SIGN;
-    // A set top bit marks a non-negative float (sign flipped), a clear one a
-    // negative float (all bits inverted).
-    if constexpr (KC == KeyClass::Float)
-      x ^= static_cast<Bits>(~(static_cast<SBits>(x) >> (NBITS - 1))) | SIGN;
-    return x;
-  }
-  __device__ static __forceinline__ Bits collapse(Bits x) {
-    if constexpr (KC == KeyClass::Float) return x == SIGN - 1 ? SIGN : x;
-    else return x;
-  }
-
-  __device__ static __forceinline__ Bits digit_source(Bits raw) { return collapse(image(raw)); }
-
-  __device__ static __forceinline__ uint32_t digit(Bits raw, uint32_t bit, uint32_t mask) {
-    return static_cast<uint32_t>(digit_source(raw) >> bit) & mask;
-  }
-  __device__ static __forceinline__ uint32_t image_digit(Bits y, uint32_t bit, uint32_t mask) {
-    return static_cast<uint32_t>(collapse(y) >> bit) & mask;
-  }
-};
 
 // Key loads of a keys-only onesweep are non-temporal: they are read once, and
 // leaving L2 to the scattered writes (whose partial lines merge there) and the
@@ -387,8 +334,6 @@ bins_scan_kernel(uint32_t *bins, uint32_t passes, uint32_t n, PassPlan *plan,
 // both modes.
 // ---------------------------------------------------------------------------
 
-enum class Rank : int { LaneAtomic = 0, MatchAny = 1 };
-
 // Items per batch of match-any ranking.
 #ifndef RCCL_RADIX_MATCH_BATCH
 #define RCCL_RADIX_MATCH_BATCH 8
@@ -530,41 +475,6 @@ __device__ __forceinline__ Desc lookback_consume(const LookbackBuf<Desc> &lbuf, 
     }
   }
   return excl;
-}
-
-// Opaque copy: the compiler must assume the value changed here, so it cannot
-// carry values derived from it across this point. Aggregate keys (record
-// rows) overload it in their own namespace, found by argument-dependent
-// lookup.
-template <class T>
-__device__ __forceinline__ void launder(T &x) {
-  asm volatile("" : "+v"(x));
-}
-
-// True when every lane of the (fully active) wave holds the same value.
-__device__ __forceinline__ bool wave_uniform(uint32_t v) {
-  return __ballot(v == __builtin_amdgcn_readfirstlane(v)) == ~uint64_t(0);
-}
-
-// Lanes of the fully active wave whose value of `d` equals this lane's, over
-// the bits set in `bits` (one ballot per bit; the digits differ in no other
-// bit).
-__device__ __forceinline__ uint64_t peer_lanes(uint32_t d, uint32_t bits) {
-  uint64_t m = ~uint64_t(0);
-#pragma unroll
-  for (int b = 0; b < 9; ++b) {
-    if (bits & (1u << b)) {
-      const bool set = ((d >> b) & 1u) != 0;
-      const uint64_t bal = __ballot(set);
-      m &= set ? bal : ~bal;
-    }
-  }
-  return m;
-}
-
-// Lowest set lane of a non-zero mask.
-__device__ __forceinline__ uint32_t lowest_lane(uint64_t m) {
-  return static_cast<uint32_t>(__builtin_ctzll(m));
 }
 
 // One tile of a onesweep pass. Keys are any trivially copyable type whose
@@ -1044,121 +954,6 @@ planned_onesweep_kernel(PlanBuffers<Bits, Val> b, size_t n, uint32_t num_tiles,
 }
 
 // ---------------------------------------------------------------------------
-// single tile: inputs of at most single_tile_items() items are sorted by one
-// block in one launch (the reference's single-tile route,
-// rccl-cub/src/radix.rs:470-492, ordering_backend/radix.rs:366-715). Keys
-// and values are loaded into LDS once; every 8-bit pass counts, scans and
-// ranks them as a onesweep tile does (per-wave counters, either ranking
-// mode) and scatters them into the other LDS buffer; the result is stored
-// once. No workspace is touched.
-// ---------------------------------------------------------------------------
-constexpr int ST_THREADS = 256;
-
-// The reference's single-tile capacity: 256 threads x 19 * 4 / max(item
-// bytes, 4) items (rccl-cub/src/workspace.rs:22-66).
-constexpr size_t single_tile_items(size_t key_bytes, size_t value_bytes) {
-  const size_t item = std::max<size_t>(std::max(key_bytes, value_bytes), 4);
-  return size_t(ST_THREADS) * std::max<size_t>(1, 19 * 4 / item);
-}
-
-template <class Bits, class Val, class Ops, int ITEMS, Rank RANK>
-__global__ void __launch_bounds__(ST_THREADS)
-single_tile_kernel(const Bits *keys_in, Bits *keys_out, const Val *vals_in, Val *vals_out,
-                   uint32_t n, uint32_t begin_bit, uint32_t end_bit) {
-  // keys_out may be keys_in (in place): every input is read before the first
-  // barrier and every output written after the last.
-  constexpr bool PAIRS = !std::is_same<Val, NoValue>::value;
-  constexpr int WAVES = ST_THREADS / 64;
-  constexpr int TILE = ST_THREADS * ITEMS;
-  constexpr int WAVE_ITEMS = 64 * ITEMS;
-  constexpr int NB = BINS + 1;
-  constexpr uint32_t DUMMY = BINS;
-  static_assert(ST_THREADS == BINS, "one thread per digit");
-  using VStore = typename std::conditional<PAIRS, Val, char>::type;
-  __shared__ Bits kbuf[2][TILE];
-  __shared__ VStore vbuf[PAIRS ? 2 : 1][PAIRS ? TILE : 1];
-  __shared__ uint32_t cnt[WAVES][NB];
-  __shared__ uint32_t wave_sum[WAVES];
-
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  for (uint32_t i = tid; i < n; i += ST_THREADS) {
-    kbuf[0][i] = keys_in[i];
-    if constexpr (PAIRS) vbuf[0][i] = vals_in[i];
-  }
-  int cur = 0;
-  for (uint32_t bit = begin_bit; bit < end_bit; bit += 8) {
-    const uint32_t mask = (1u << min(8u, end_bit - bit)) - 1u;
-    for (uint32_t i = tid; i < WAVES * NB; i += ST_THREADS) (&cnt[0][0])[i] = 0;
-    __syncthreads();
-    // (wave, item, lane) order is source order; items at or past n are
-    // dummies, placed after every key.
-    Bits key[ITEMS];
-    uint32_t dg[ITEMS];
-    uint32_t *wcnt = cnt[wave];
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const uint32_t i = wave * WAVE_ITEMS + uint32_t(j) * 64 + lane;
-      key[j] = kbuf[cur][min(i, uint32_t(TILE - 1))];
-      dg[j] = i < n ? Ops::digit(key[j], bit, mask) : DUMMY;
-      __hip_atomic_fetch_add(&wcnt[dg[j]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __syncthreads();
-    // Digit starts (exclusive scan over digits), then each wave's start.
-    uint32_t wc[WAVES], count = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      wc[w] = cnt[w][tid];
-      count += wc[w];
-    }
-    const uint32_t inc = wave_inclusive_sum(count, lane);
-    if (lane == 63) wave_sum[wave] = inc;
-    __syncthreads();
-    uint32_t run = inc - count;
-    for (uint32_t w = 0; w < wave; ++w) run += wave_sum[w];
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      cnt[w][tid] = run;
-      run += wc[w];
-    }
-    if (tid < WAVES) cnt[tid][DUMMY] = max(n, tid * uint32_t(WAVE_ITEMS));
-    __syncthreads();
-    const uint32_t dbits = mask | DUMMY;
-#pragma unroll
-    for (int j = 0; j < ITEMS; ++j) {
-      const uint32_t d = dg[j];
-      uint32_t pos;
-      if constexpr (RANK == Rank::MatchAny) {
-        const uint64_t m = peer_lanes(d, dbits);
-        const uint32_t below = popc_below(m);
-        const uint32_t base =
-            below == 0 ? __hip_atomic_fetch_add(&wcnt[d],
-                                                static_cast<uint32_t>(__builtin_popcountll(m)),
-                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                       : 0u;
-        pos = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(
-                  static_cast<int>(lowest_lane(m) << 2), static_cast<int>(base))) +
-              below;
-      } else {
-        pos = __hip_atomic_fetch_add(&wcnt[d], 1u, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      pos = min(pos, uint32_t(TILE - 1));
-      kbuf[cur ^ 1][pos] = key[j];
-      if constexpr (PAIRS) {
-        const uint32_t i = wave * WAVE_ITEMS + uint32_t(j) * 64 + lane;
-        vbuf[cur ^ 1][pos] = vbuf[cur][min(i, uint32_t(TILE - 1))];
-      }
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-  for (uint32_t i = tid; i < n; i += ST_THREADS) {
-    keys_out[i] = kbuf[cur][i];
-    if constexpr (PAIRS) vals_out[i] = vbuf[cur][i];
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
 
@@ -1282,31 +1077,82 @@ rccl_hip_status launch_onesweeps(SortArgs &a, const Layout &l, uint32_t passes,
   return ok();
 }
 
+// A short sort (short_sort): one block, or block-sorted tiles and their
+// rank merge. The result lands where the other routes leave it: a planned
+// sort's in its output, a plain one's in the buffer that its passes' flips end
+// in (one flip for the reference's single-tile sizes, else one per pass).
 template <class Bits, class Val, class Ops, Rank RANK>
-rccl_hip_status launch_single_tile(SortArgs &a) {
+rccl_hip_status launch_short(SortArgs &a, const Layout &l, uint32_t passes) {
   constexpr size_t VBYTES = std::is_same<Val, NoValue>::value ? 0 : sizeof(Val);
-  constexpr int ITEMS = static_cast<int>(single_tile_items(sizeof(Bits), VBYTES) / ST_THREADS);
-  const int dst = a.single_to_other ? 1 - a.cur : a.cur;
-  {
-    KernelTimer t("radix_single_tile", a.stream, a.n);
-    single_tile_kernel<Bits, Val, Ops, ITEMS, RANK><<<1, ST_THREADS, 0, a.stream>>>(
-        static_cast<const Bits *>(a.keys[a.cur]), static_cast<Bits *>(a.keys[dst]),
-        static_cast<const Val *>(a.vals[a.cur]), static_cast<Val *>(a.vals[dst]),
-        static_cast<uint32_t>(a.n), a.begin_bit, a.end_bit);
+  const bool from_src = a.src_keys != nullptr;
+  const void *kin = from_src ? a.src_keys : a.keys[a.cur];
+  const void *vin = from_src ? a.src_vals : a.vals[a.cur];
+  int dst = 0;
+  if (!a.planned) {
+    const bool flip = a.n <= single_tile_items(sizeof(Bits), VBYTES) ? a.single_to_other
+                                                                     : (passes & 1u) != 0;
+    dst = flip ? 1 - a.cur : a.cur;
   }
-  RCCL_HIP_TRY(check_launch("radix single tile"));
+  const uint32_t n = static_cast<uint32_t>(a.n);
+  const uint32_t tile = static_cast<uint32_t>(short_tile(sizeof(Bits), a.n));
+  if (a.n <= tile) {
+    KernelTimer t("radix_single_tile", a.stream, a.n);
+    block_sort_kernel<Bits, Val, Ops, BLOCK_ITEMS, RANK><<<1, BLOCK_THREADS, 0, a.stream>>>(
+        static_cast<const Bits *>(kin), static_cast<Bits *>(a.keys[dst]),
+        static_cast<const Val *>(vin), static_cast<Val *>(a.vals[dst]), n, n, a.begin_bit,
+        a.end_bit, nullptr);
+    a.cur = dst;
+    return check_launch("radix single tile");
+  }
+  // The tiles go to the buffer that the result does not end in.
+  const int mid = 1 - dst;
+  const uint32_t tiles = (n + tile - 1) / tile;
+  // A planned sort's workspace ends with the samples; a plain one's are in the
+  // place of the look-back buffers, which these sorts don't use.
+  const size_t sample_bytes = short_sample_bytes(sizeof(Bits), a.n);
+  Bits *samples =
+      reinterpret_cast<Bits *>(a.ws + (a.planned ? l.total + plan_bytes() : l.lb[0]));
+  if (!a.planned && sample_bytes > 2 * l.lb_bytes)
+    return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "radix sample space", sample_bytes,
+                     2 * l.lb_bytes);
+  {
+    KernelTimer t("radix_block_sort", a.stream, a.n);
+    block_sort_kernel<Bits, Val, Ops, BLOCK_ITEMS, RANK><<<tiles, BLOCK_THREADS, 0, a.stream>>>(
+        static_cast<const Bits *>(kin), static_cast<Bits *>(a.keys[mid]),
+        static_cast<const Val *>(vin), static_cast<Val *>(a.vals[mid]), n, tile, a.begin_bit,
+        a.end_bit, samples);
+  }
+  RCCL_HIP_TRY(check_launch("radix block sort"));
+  {
+    KernelTimer t("radix_rank_merge", a.stream, a.n);
+    const auto merge = [&](auto tile_const) {
+      constexpr uint32_t TILE = decltype(tile_const)::value;
+      const size_t slots = (tiles + RM_WAYS - 1) / RM_WAYS * RM_WAYS * (TILE / SAMPLE);
+      rank_merge_kernel<Bits, Val, Ops, TILE>
+          <<<(n + RM_THREADS - 1) / RM_THREADS, RM_THREADS, slots * sizeof(Bits), a.stream>>>(
+              static_cast<const Bits *>(a.keys[mid]), static_cast<Bits *>(a.keys[dst]),
+              static_cast<const Val *>(a.vals[mid]), static_cast<Val *>(a.vals[dst]), n, tiles,
+              a.begin_bit, a.end_bit, samples);
+    };
+    if (tile == RM_TILE_SMALL) merge(std::integral_constant<uint32_t, RM_TILE_SMALL>{});
+    else merge(std::integral_constant<uint32_t, RM_TILE_LARGE>{});
+  }
   a.cur = dst;
-  return ok();
+  return check_launch("radix rank merge");
 }
 
 template <class Bits, class Val, class Ops, class Desc>
 rccl_hip_status run_passes(SortArgs &a, const Layout &l, uint32_t passes) {
-  DeviceCaps caps;
-  RCCL_HIP_TRY(device_caps(&caps, a.stream));
   constexpr size_t VBYTES = std::is_same<Val, NoValue>::value ? 0 : sizeof(Val);
-  if (!a.planned && !a.src_keys && a.n <= single_tile_items(sizeof(Bits), VBYTES))
-    return caps.rank == Rank::LaneAtomic ? launch_single_tile<Bits, Val, Ops, Rank::LaneAtomic>(a)
-                                         : launch_single_tile<Bits, Val, Ops, Rank::MatchAny>(a);
+  DeviceCaps caps;
+  const rccl_hip_status probed = device_caps(&caps, a.stream);
+  // Comparator sorts below COMPARATOR_MIN_ITEMS need nothing of the device:
+  // without its probe they rank by match-any.
+  if (probed != RCCL_HIP_SUCCESS && !(a.planned && a.n < COMPARATOR_MIN_ITEMS)) return probed;
+  if (short_sort(a.n))
+    return probed == RCCL_HIP_SUCCESS && caps.rank == Rank::LaneAtomic
+               ? launch_short<Bits, Val, Ops, Rank::LaneAtomic>(a, l, passes)
+               : launch_short<Bits, Val, Ops, Rank::MatchAny>(a, l, passes);
   uint32_t *bins = reinterpret_cast<uint32_t *>(a.ws + l.bins);
   uint32_t *skew = reinterpret_cast<uint32_t *>(a.ws + l.skew);
   {

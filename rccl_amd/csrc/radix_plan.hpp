@@ -133,6 +133,50 @@ constexpr bool small_tiles(size_t key_bytes, size_t value_bytes, size_t n, bool 
                                                                                value_bytes);
 }
 
+// Short sorts (radix_block_kernels.hpp): one block sorts its tile in LDS, up
+// to 16 such tiles are then merged by rank; one or two launches where the
+// onesweep takes three and one per key byte. A block is as wide as the CU
+// allows. us per sort (a copy of the keys included), onesweep -> here:
+//   u32 keys         2^14 38.4 -> 17.5   2^16 43.8 -> 25.4   2^17 44.5 -> 34.4
+//   u64 + u32 pairs  2^14 63.2 -> 28.0   2^16 75.8 -> 36.9   2^17 78.7 -> 52.3
+//   f32 + 8 B pairs  2^14 39.6 -> 22.1   2^16 44.2 -> 30.6   2^17 46.1 -> 44.2
+// The rank merge's work grows with items x tiles: at 2^18 it loses (u32 keys
+// 45 -> 65, u64 + u32 pairs 87 -> 98).
+constexpr int BLOCK_THREADS = 1024;
+constexpr int BLOCK_ITEMS = 8;  // per thread: tiles of at most 8,192 items
+constexpr size_t SHORT_ITEMS = 131072;
+constexpr uint32_t SAMPLE = 32;     // sorted items per sample of a tile
+constexpr int RM_THREADS = 256;     // items per rank-merge block
+constexpr int RM_WAYS = 4;          // tiles searched at once
+constexpr size_t RM_TILE_SMALL = 4096, RM_TILE_LARGE = 8192;
+constexpr bool short_sort(size_t n) { return n <= SHORT_ITEMS; }
+// Tile of a short sort. One block alone holds the sort up to where a second
+// launch costs less than its longer passes: 8,192 items for 4-byte keys (one
+// block 18 us, two launches 17.5), 5,120 for 8-byte keys with their eight
+// passes (27.6 and 28.0; at 8,192 one block takes 32.4). Rank-merged tiles are
+// the smaller ones while those make at most 16 (u64 + u32 pairs at 2^16 36.9
+// against 41.6 us, at 2^17 54.3 against 52.3).
+constexpr size_t short_tile(size_t key_bytes, size_t n) {
+  return n <= (key_bytes > 4 ? 5120 : RM_TILE_LARGE)
+             ? RM_TILE_LARGE
+             : (n <= 16 * RM_TILE_SMALL ? RM_TILE_SMALL : RM_TILE_LARGE);
+}
+// Samples of a short sort's tiles.
+inline size_t short_sample_bytes(size_t key_bytes, size_t n) {
+  return short_sort(n) ? align_up((n + SAMPLE - 1) / SAMPLE * key_bytes, 256) : 0;
+}
+// The reference's single-tile capacity: 256 threads x 19 * 4 / max(item
+// bytes, 4) items (rccl-cub/src/workspace.rs:22-66). A DoubleBuffer sort up to
+// it flips the selector once.
+constexpr size_t single_tile_items(size_t key_bytes, size_t value_bytes) {
+  return 256 * (19 * 4 / (stage_elem(key_bytes, value_bytes) > 4
+                              ? stage_elem(key_bytes, value_bytes)
+                              : 4));
+}
+// Comparator sorts (DeviceMergeSort) of fewer items also run on a device that
+// was not probed, under graph capture too.
+constexpr size_t COMPARATOR_MIN_ITEMS = 65536;
+
 // Pass plan of a sort that skips trivial passes (one digit holds every key:
 // the pass would not move anything). Buffers: 0 the input, 1 the output,
 // 2 the scratch; lb is the look-back buffer of the pass (the active passes

@@ -1,0 +1,128 @@
+"""Short sorts (one block, or block-sorted tiles and their rank merge) against
+the oracle, at the edges of their tiles and routes."""
+import numpy as np
+import pytest
+
+import oracle
+from rccl_amd import cub, workloads
+from rccl_amd.device import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+
+# Rows of a block (1,024), one block / rank merge (5,120 for 8-byte keys,
+# 8,192 for 4-byte), tile ends (4,096), the larger tiles (65,536) and the onesweep.
+SIZES = [1, 1_023, 1_025, 5_120, 5_121, 8_191, 8_192, 8_193, 12_289, 65_535, 65_536, 65_537,
+         131_071, 131_072, 131_073]
+
+
+def _keys(kind, n, dist, seed):
+    dt = np.dtype(oracle.KIND_DTYPES[kind])
+    bits = workloads.hash_range(seed, n) >> np.uint64(64 - 8 * dt.itemsize)
+    if dist == "ties":  # few values, the largest and the smallest image among them
+        bits = bits % np.uint64(5)
+        bits[bits == 4] = np.uint64((1 << (8 * dt.itemsize)) - 1)
+    elif dist == "sorted":
+        bits = np.sort(bits)
+    elif dist == "low":  # constant high bytes
+        bits = bits & np.uint64(0x3FFF)
+    bits = bits.astype(f"u{dt.itemsize}")
+    if dt.kind == "f":
+        bits[::7] = 0
+        bits[1::11] = 1 << (8 * dt.itemsize - 1)
+    return bits.view(dt)
+
+
+def _values(width, n):
+    if width == 16:
+        return workloads.hash_range(99, 2 * n).view(np.dtype((np.void, 16)))
+    return (np.arange(n, dtype=np.uint64) % np.uint64(1 << (8 * width - 1))).astype(f"u{width}")
+
+
+def _equal(a, b):
+    return np.array_equal(np.ascontiguousarray(a).view(np.uint8),
+                          np.ascontiguousarray(b).view(np.uint8))
+
+
+@pytest.mark.parametrize("kind,width,descending", [
+    ("u32", 0, False), ("u32", 4, True), ("f32", 8, True), ("i32", 16, False), ("u64", 0, True),
+    ("u64", 4, False), ("f64", 2, False), ("i64", 8, False)])
+@pytest.mark.parametrize("n", SIZES)
+def test_short_sorts(launch, radix_ranking, kind, width, descending, n):
+    for dist in ("uniform", "ties", "sorted", "low"):
+        host = _keys(kind, n, dist, 7 * n + width)
+        keys = DeviceBuffer.from_host(host)
+        if width:
+            vals_h = _values(width, n)
+            vals = DeviceBuffer.from_host(vals_h)
+            ws = cub.device_radix_sort_pairs_workspace(launch, host.dtype, vals_h.dtype, n)
+            (cub.device_radix_sort_pairs_descending if descending
+             else cub.device_radix_sort_pairs)(launch, keys, vals, ws)
+            launch.synchronize()
+            wk, wv = oracle.radix_sort(kind, host, vals_h, descending=descending)
+            assert _equal(vals.to_host_vec(), wv), dist
+        else:
+            ws = cub.device_radix_sort_workspace(launch, host.dtype, n)
+            (cub.device_radix_sort_keys_descending if descending
+             else cub.device_radix_sort_keys)(launch, keys, ws)
+            launch.synchronize()
+            wk = oracle.radix_sort(kind, host, descending=descending)
+        assert _equal(keys.to_host_vec(), wk), dist
+
+
+@pytest.mark.parametrize("kind,window", [("u32", (0, 24)), ("u32", (5, 30)), ("u32", (31, 32)),
+                                         ("u64", (3, 64)), ("u64", (27, 37)), ("f64", (20, 61))])
+@pytest.mark.parametrize("n", [6_000, 70_001])
+@pytest.mark.parametrize("second", [False, True])
+def test_short_windows_and_selector(launch, radix_ranking, kind, window, n, second):
+    """Bit windows (across the key's words too), and the selector of the
+    DoubleBuffer form: one flip per pass, whichever half holds the input."""
+    host, vals_h = _keys(kind, n, "uniform", n), np.arange(n, dtype=np.uint32)
+    k = [DeviceBuffer.from_host(host), DeviceBuffer.zeroed(host.dtype, n)]
+    v = [DeviceBuffer.from_host(vals_h), DeviceBuffer.zeroed(np.uint32, n)]
+    if second:
+        k, v = k[::-1], v[::-1]
+    buffers = cub.DoubleBuffer((k[0], v[0]), (k[1], v[1]), current_is_first=not second)
+    ws = cub.device_radix_sort_pairs_buffer_workspace(launch, host.dtype, np.uint32, n)
+    cub.device_radix_sort_pairs_buffer(launch, buffers, range(*window), ws)
+    launch.synchronize()
+    passes = (window[1] - window[0] + 7) // 8
+    assert buffers.current_is_first() == ((passes % 2 == 0) != second)
+    wk, wv = oracle.radix_sort(kind, host, vals_h, begin_bit=window[0], end_bit=window[1])
+    ck, cv = buffers.current()
+    assert _equal(ck.to_host_vec(), wk) and _equal(cv.to_host_vec(), wv)
+
+
+@pytest.mark.parametrize("kind,width", [("u32", 0), ("f32", 4), ("u64", 8), ("i64", 16)])
+@pytest.mark.parametrize("n", [1, 8_193, 50_001, 65_537, 131_072])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_short_comparator_sorts(launch, radix_ranking, kind, width, n, in_place):
+    """DeviceMergeSort of 4- and 8-byte keys takes the same kernels: stable,
+    copy forms leaving their input alone."""
+    host = _keys(kind, n, "ties", 3 * n)
+    if host.dtype.kind == "f":
+        host = np.where(np.isnan(host), host.dtype.type(-1.5), host)
+    keys = DeviceBuffer.from_host(host)
+    out = keys if in_place else DeviceBuffer.zeroed(host.dtype, n)
+    order = np.argsort(-host.astype(np.float64) if host.dtype.kind == "f"
+                       else ~host, kind="stable")  # descending
+    if width:
+        vals_h = _values(width, n)
+        vals = DeviceBuffer.from_host(vals_h)
+        outv = vals if in_place else DeviceBuffer.zeroed(vals_h.dtype, n)
+        ws = cub.device_merge_sort_pairs_workspace(launch, host.dtype, vals_h.dtype, n)
+        if in_place:
+            cub.device_merge_sort_pairs(launch, keys, vals, ws, cub.descending)
+        else:
+            cub.device_merge_sort_pairs_copy(launch, keys, vals, ws, out, outv, cub.descending)
+        launch.synchronize()
+        assert _equal(outv.to_host_vec(), vals_h[order])
+    else:
+        ws = cub.device_merge_sort_workspace(launch, host.dtype, n)
+        if in_place:
+            cub.device_merge_sort_keys(launch, keys, ws, cub.descending)
+        else:
+            cub.device_merge_sort_keys_copy(launch, keys, ws, out, cub.descending)
+        launch.synchronize()
+    assert _equal(out.to_host_vec(), host[order])
+    if not in_place:
+        assert _equal(keys.to_host_vec(), host)
