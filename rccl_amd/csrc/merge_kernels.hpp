@@ -95,22 +95,28 @@ constexpr size_t call_tile_items(size_t total) {
 }
 
 // Splits for tile boundaries 0..tiles: splits[t] = A items among the first
-// min(t * tile, na + nb) merged outputs.
-template <class K, class Cmp>
+// min(t * tile, na + nb) merged outputs. G lanes search each boundary
+// (ordering::group_merge_path); G == 1 searches by itself.
+template <class K, class Cmp, uint32_t G>
 __global__ void __launch_bounds__(256)
 partition_kernel(const K *__restrict__ a, size_t na, const K *__restrict__ b, size_t nb,
                  size_t tile, size_t count, uint64_t *__restrict__ splits) {
-  const size_t t = size_t(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= count) return;
+  const size_t t = (size_t(blockIdx.x) * 256 + threadIdx.x) / G;
+  if (t >= count) return;  // whole groups
   const size_t diag = std::min(t * tile, na + nb);
-  splits[t] = ordering::merge_path<K>([&](size_t i) { return a[i]; }, na,
-                                      [&](size_t j) { return b[j]; }, nb, diag, Cmp{});
+  const auto ra = [&](size_t i) { return a[i]; };
+  const auto rb = [&](size_t j) { return b[j]; };
+  size_t i;
+  if constexpr (G > 1) i = ordering::group_merge_path<G, K>(ra, na, rb, nb, diag, Cmp{});
+  else i = ordering::merge_path<K>(ra, na, rb, nb, diag, Cmp{});
+  if (threadIdx.x % G == 0) splits[t] = i;
 }
 
-// Sampled partition (integer keys, from SAMPLED_MIN_TILES tiles):
+// Sampled partition (integer keys, from ordering::PARTITION_SAMPLED_MIN tiles):
 // ordering::merge_sample_kernel, then each tile boundary's split from
 // ordering::sampled_merge_path.
-constexpr size_t SAMPLED_MIN_TILES = 512;
+// The workspace holds the samples from fewer tiles on.
+constexpr size_t WORKSPACE_SAMPLED_MIN = 512;
 
 template <class K, class Cmp>
 __global__ void __launch_bounds__(256)
@@ -240,16 +246,16 @@ struct MergeArgs {
   hipStream_t stream;
 };
 
-// The sampled partition serves merges of at least SAMPLED_MIN_TILES tiles.
+// Whether a merge of at least min_tiles tiles, with samples.
 template <class K, class V>
-bool use_sampled(size_t na, size_t nb) {
+bool sampled_from(size_t na, size_t nb, size_t min_tiles) {
   const size_t tile = call_tile_items<K, V>(na + nb);
   const size_t tiles = (na + nb + tile - 1) / tile;
-  return ordering::sampled_partition_for<K>() && na > 0 && nb > 0 && tiles >= SAMPLED_MIN_TILES;
+  return ordering::sampled_partition_for<K>() && na > 0 && nb > 0 && tiles >= min_tiles;
 }
 
 // Splits (one u64 per tile boundary), then the samples' m_k (one u32 per
-// MERGE_SAMPLE items of A) when the sampled partition runs.
+// MERGE_SAMPLE items of A) from WORKSPACE_SAMPLED_MIN tiles.
 template <class K, class V>
 size_t workspace_bytes(size_t na, size_t nb) {
   const size_t total = na + nb;
@@ -257,7 +263,7 @@ size_t workspace_bytes(size_t na, size_t nb) {
   const size_t tile = call_tile_items<K, V>(total);
   const size_t tiles = (total + tile - 1) / tile;
   size_t bytes = align_up((tiles + 1) * sizeof(uint64_t), 256);
-  if (use_sampled<K, V>(na, nb)) bytes += align_up(ordering::merge_samples(na) * 4, 256);
+  if (sampled_from<K, V>(na, nb, WORKSPACE_SAMPLED_MIN)) bytes += align_up(ordering::merge_samples(na) * 4, 256);
   return bytes;
 }
 
@@ -271,7 +277,7 @@ rccl_hip_status run_merge_shape(const MergeArgs &m) {
   const size_t tiles = (total + TILE - 1) / TILE;
   uint64_t *splits = static_cast<uint64_t *>(m.ws);
   const dim3 pgrid(static_cast<uint32_t>((tiles + 1 + 255) / 256));
-  if (use_sampled<K, V>(m.na, m.nb)) {
+  if (sampled_from<K, V>(m.na, m.nb, ordering::PARTITION_SAMPLED_MIN)) {
     uint32_t *samples = reinterpret_cast<uint32_t *>(static_cast<unsigned char *>(m.ws) +
                                                      align_up((tiles + 1) * sizeof(uint64_t), 256));
     const size_t ka = ordering::merge_samples(m.na);
@@ -289,9 +295,14 @@ rccl_hip_status run_merge_shape(const MergeArgs &m) {
         samples, splits);
   } else {
     KernelTimer t("merge_partition", m.stream, tiles + 1);
-    partition_kernel<K, Cmp><<<pgrid, 256, 0, m.stream>>>(static_cast<const K *>(m.a), m.na,
-                                                          static_cast<const K *>(m.b), m.nb, TILE,
-                                                          tiles + 1, splits);
+    const auto partition = [&](auto lanes) {
+      constexpr uint32_t G = decltype(lanes)::value;
+      partition_kernel<K, Cmp, G>
+          <<<dim3(static_cast<uint32_t>(((tiles + 1) * G + 255) / 256)), 256, 0, m.stream>>>(
+              static_cast<const K *>(m.a), m.na, static_cast<const K *>(m.b), m.nb, TILE,
+              tiles + 1, splits);
+    };
+    ordering::with_partition_lanes<K>(tiles, partition);
   }
   RCCL_HIP_TRY(check_launch("merge partition"));
   {

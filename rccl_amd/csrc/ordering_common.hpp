@@ -136,35 +136,67 @@ __host__ __device__ inline size_t merge_samples(size_t na) { return (na + MERGE_
 
 // ---------------------------------------------------------------------------
 // Group searches. A search over HBM whose every probe is a dependent round
-// trip is latency-bound. The searches below run on the 8 lanes of an aligned
-// lane group, which all hold the same search: each round the lanes probe 8
+// trip is latency-bound. The searches below run on the G lanes of an aligned
+// lane group, which all hold the same search: each round the lanes probe G
 // evenly spaced points and a ballot counts those still before the answer, a
-// 9-ary search: about log9 of the range in dependent rounds instead of log2.
+// (G + 1)-ary search: log2 / log2(G + 1) of a binary search's dependent rounds.
 // ---------------------------------------------------------------------------
 constexpr uint32_t SEARCH_GROUP = 8;
 
 // First x in [lo, hi) with !before(x), or hi, where `before` holds on a
 // prefix of the range (on any other predicate the result stays in [lo, hi]).
 // Every lane of the group calls it with the same arguments.
-template <class Before>
+template <uint32_t G = SEARCH_GROUP, class Before>
 __device__ __forceinline__ size_t group_first_not(size_t lo, size_t hi, Before before) {
+  static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0, "lanes of an aligned group");
   const uint32_t lane = lane_id();
-  const uint32_t sub = lane & (SEARCH_GROUP - 1u), base = lane & ~(SEARCH_GROUP - 1u);
+  const uint32_t sub = lane & (G - 1u), base = lane & ~(G - 1u);
+  const auto count = [&](bool bf) {
+    return static_cast<size_t>(
+        __builtin_popcountll((__ballot(bf) >> base) & (~uint64_t(0) >> (64 - G))));
+  };
   while (lo < hi) {
     const size_t span = hi - lo;
-    if (span <= SEARCH_GROUP) {
-      const bool bf = sub < span && before(lo + sub);
-      return lo + __builtin_popcount(static_cast<uint32_t>(__ballot(bf) >> base) & 0xFFu);
-    }
-    const bool bf = before(lo + (size_t(sub) + 1) * span / 9);
-    const size_t cnt = __builtin_popcount(static_cast<uint32_t>(__ballot(bf) >> base) & 0xFFu);
-    // Probe j sits at lo + (j + 1) * span / 9: the answer lies after probe
-    // cnt - 1 and at or before probe cnt.
+    if (span <= G) return lo + count(sub < span && before(lo + sub));
+    const size_t cnt = count(before(lo + (size_t(sub) + 1) * span / (G + 1)));
+    // Probe j sits at lo + (j + 1) * span / (G + 1): the answer lies after
+    // probe cnt - 1 and at or before probe cnt.
     const size_t l0 = lo;
-    if (cnt > 0) lo = l0 + cnt * span / 9 + 1;
-    if (cnt < SEARCH_GROUP) hi = l0 + (cnt + 1) * span / 9;
+    if (cnt > 0) lo = l0 + cnt * span / (G + 1) + 1;
+    if (cnt < G) hi = l0 + (cnt + 1) * span / (G + 1);
   }
   return lo;
+}
+
+// merge_path of diagonal `diag` by the G lanes of a group (integer keys: with
+// NaN the predicate is no prefix). Every lane returns the split.
+template <uint32_t G, class K, class Cmp, class ReadA, class ReadB>
+__device__ __forceinline__ size_t group_merge_path(ReadA a, size_t na, ReadB b, size_t nb,
+                                                   size_t diag, Cmp less) {
+  return group_first_not<G>(diag > nb ? diag - nb : 0, diag < na ? diag : na,
+                            [&](size_t i) { return !less(b(diag - 1 - i), a(i)); });
+}
+
+// Calls run(std::integral_constant<uint32_t, lanes>) with the lanes per tile
+// boundary of a partition that searches the whole inputs. Integer keys of few
+// boundaries take a wave each (three or four rounds instead of 16 to 22), more
+// of them 16 and then 8 lanes; from PARTITION_SAMPLED_MIN they are bound by
+// their line reads and take the samples (u32 pairs, us per merge, before ->
+// here: 2^20 outputs 18.1 -> 12.6, 2^22 27.3 -> 20.1, 2^24 75.9 -> 69.8; 2^25
+// 127.6 sampled, 130.4 with eight lanes). Floats keep one lane.
+#ifndef RCCL_PARTITION_SAMPLED_MIN
+#define RCCL_PARTITION_SAMPLED_MIN 16384
+#endif
+constexpr size_t PARTITION_SAMPLED_MIN = RCCL_PARTITION_SAMPLED_MIN;
+template <class K, class Run>
+void with_partition_lanes(size_t tiles, Run run) {
+  if constexpr (!sampled_partition_for<K>()) {
+    run(std::integral_constant<uint32_t, 1>{});
+  } else {
+    if (tiles < 256) run(std::integral_constant<uint32_t, 64>{});
+    else if (tiles < 2048) run(std::integral_constant<uint32_t, 16>{});
+    else run(std::integral_constant<uint32_t, SEARCH_GROUP>{});
+  }
 }
 
 // Eight lanes per sample (group_first_not): with one sample per 2,048 items

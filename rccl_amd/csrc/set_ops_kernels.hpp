@@ -30,6 +30,9 @@ using ordering::NoValue;
 #ifndef RCCL_SET_THREADS
 #define RCCL_SET_THREADS 512
 #endif
+#ifndef RCCL_SET_ITEMS_4B
+#define RCCL_SET_ITEMS_4B 24
+#endif
 #ifndef RCCL_SET_ITEMS_8B
 #define RCCL_SET_ITEMS_8B 16
 #endif
@@ -50,36 +53,74 @@ constexpr uint32_t XCD_RUN = RCCL_SET_XCD_RUN;  // tiles per XCD run (xcd_order_
 
 enum Op : int { UNION = 0, INTERSECTION = 1, DIFFERENCE = 2, SYMMETRIC_DIFFERENCE = 3 };
 
-// Union and symmetric difference of 8-byte keys emit from both inputs: their
-// outputs, kept in registers for two partition tiles, fit the 128-register
-// budget without spilling at one item fewer per thread.
+// Tile shapes. Large inputs: two partition tiles per block and look-back tile
+// (SUB_TILES), as many items per thread as two tiles' outputs leave registers
+// for without spilling (128 per thread, two blocks per CU). More items mean
+// fewer look-backs: keys only, 6 x 10^7 u32 keys, 16 -> 24 items: union 198 ->
+// 174 us, intersection 174 -> 152. Values are not staged, so their width plays
+// no part.
+// Small inputs: one partition tile per block, so that they still spread over
+// the CUs (u32 keys, union, one / two tiles per block: 3 x 10^4 keys 13.8 /
+// 21.2 us, 5 x 10^5 15.7 / 23.3, 4 x 10^6 29.6 / 36). They end where the
+// blocks no longer fit the chip at once: 640 tiles for 4-byte keys, 448 for
+// 8-byte keys (4.2 x 10^6 keys, 513 tiles: 38.1 against 34.6 us).
 #ifndef RCCL_SET_ITEMS_8B_BOTH
 #define RCCL_SET_ITEMS_8B_BOTH 15
 #endif
-template <class K, class V, int OP>
-constexpr int items_for() {
-  constexpr bool keys_only = std::is_same<V, NoValue>::value;
-  constexpr size_t bytes = sizeof(K) + (keys_only ? 0 : sizeof(V));
-  if constexpr (keys_only && sizeof(K) == 8 && (OP == UNION || OP == SYMMETRIC_DIFFERENCE))
-    return RCCL_SET_ITEMS_8B_BOTH;
-  return bytes <= 8 ? RCCL_SET_ITEMS_8B : (bytes <= 16 ? 12 : 8);
-}
-// The fewest items per thread over the four operations: the most partition
-// tiles, which sizes a workspace that serves every operation.
-template <class K, class V>
-constexpr int min_items_for() {
-  return std::min(std::min(items_for<K, V, UNION>(), items_for<K, V, INTERSECTION>()),
-                  std::min(items_for<K, V, DIFFERENCE>(), items_for<K, V, SYMMETRIC_DIFFERENCE>()));
-}
-// Partition tiles per block (and per look-back tile): two for keys only,
-// whose two register sets of outputs fit; one where values double them.
+#ifndef RCCL_SET_ITEMS_8B_PAIRS
+#define RCCL_SET_ITEMS_8B_PAIRS 12
+#endif
+#ifndef RCCL_SET_ITEMS_4B_BOTH
+#define RCCL_SET_ITEMS_4B_BOTH 16
+#endif
+#ifndef RCCL_SET_ITEMS_4B_PAIRS
+#define RCCL_SET_ITEMS_4B_PAIRS 20
+#endif
 #ifndef RCCL_SET_SUB_TILES
 #define RCCL_SET_SUB_TILES 2
 #endif
-template <class K, class V>
-constexpr int sub_tiles_for() {
-  return std::is_same<V, NoValue>::value ? RCCL_SET_SUB_TILES : 1;
+constexpr int SUB_TILES = RCCL_SET_SUB_TILES;
+template <class K, class V, int OP>
+constexpr int items_for() {
+  constexpr bool both = OP == UNION || OP == SYMMETRIC_DIFFERENCE;
+  constexpr bool pairs = !std::is_same<V, NoValue>::value;
+  if constexpr (sizeof(K) < 8)
+    return pairs ? (both ? RCCL_SET_ITEMS_4B_BOTH : RCCL_SET_ITEMS_4B_PAIRS) : RCCL_SET_ITEMS_4B;
+  if constexpr (pairs) return RCCL_SET_ITEMS_8B_PAIRS - (both ? 1 : 0);
+  return both ? RCCL_SET_ITEMS_8B_BOTH : RCCL_SET_ITEMS_8B;
 }
+// (14 items of 8-byte keys with values: two blocks' tiles fit the LDS.)
+template <class K, class V>
+constexpr int small_items_for() {
+  return sizeof(K) == 8 && !std::is_same<V, NoValue>::value ? 14 : 16;
+}
+template <class K, class V>
+constexpr bool small_shape(size_t total) {
+  return total <= size_t(sizeof(K) < 8 ? 640 : 448) * THREADS * small_items_for<K, V>();
+}
+
+// Splits of one-tile blocks are 32-bit (their inputs end far below 2^32): with
+// one look-back tile per partition tile they then fit the workspace.
+template <int SUB>
+using Split = typename std::conditional<SUB == 1, uint32_t, uint64_t>::type;
+
+// What a workspace is sized for, whatever shape runs in it: partition tiles of
+// these many items per thread, two per look-back tile for keys only, 64-bit
+// splits, and samples from WORKSPACE_SAMPLED_MIN tiles. The shapes above take
+// no more.
+template <class K, class V, int OP>
+constexpr int workspace_items_for() {
+  constexpr bool keys_only = std::is_same<V, NoValue>::value;
+  constexpr size_t bytes = sizeof(K) + (keys_only ? 0 : sizeof(V));
+  if constexpr (keys_only && sizeof(K) == 8 && (OP == UNION || OP == SYMMETRIC_DIFFERENCE))
+    return 15;
+  return bytes <= 8 ? 16 : (bytes <= 16 ? 12 : 8);
+}
+template <class V>
+constexpr int workspace_sub_tiles() {
+  return std::is_same<V, NoValue>::value ? 2 : 1;
+}
+constexpr size_t WORKSPACE_SAMPLED_MIN = 512;
 
 // Finite arithmetic input range: item i is start + step * i in the key's own
 // wrapping integer arithmetic (rccl-cub/src/ordering_backend/set.rs:49-81,
@@ -217,16 +258,18 @@ __device__ __forceinline__ void balanced_path(RA a, size_t na, RB b, size_t nb, 
 // the ticket: `state_words` words at `state`), which no earlier launch of the
 // call touches, so no separate clearing launch is needed.
 // With SAMPLED, the merge-path split comes from the samples of
-// ordering::merge_sample_kernel (m) before the balanced path adjusts it.
-template <class K, class Cmp, bool ARITH, bool SAMPLED>
+// ordering::merge_sample_kernel (m) before the balanced path adjusts it;
+// otherwise G lanes search for it (one by itself), and each of them adjusts it.
+template <class K, class Cmp, class S, bool ARITH, bool SAMPLED, uint32_t G>
 __global__ void __launch_bounds__(256)
 partition_kernel(const K *__restrict__ a, size_t na, const K *__restrict__ b, size_t nb,
-                 size_t tile, size_t count, uint64_t *__restrict__ splits, Arith<K> ar,
+                 size_t tile, size_t count, S *__restrict__ splits, Arith<K> ar,
                  Arith<K> br, uint64_t *__restrict__ state, size_t state_words,
                  const uint32_t *__restrict__ m) {
-  const size_t t = size_t(blockIdx.x) * 256 + threadIdx.x;
-  for (size_t w = t; w < state_words; w += size_t(gridDim.x) * 256) state[w] = 0;
-  if (t >= count) return;
+  const size_t thread = size_t(blockIdx.x) * 256 + threadIdx.x;
+  for (size_t w = thread; w < state_words; w += size_t(gridDim.x) * 256) state[w] = 0;
+  const size_t t = thread / G;
+  if (t >= count) return;  // whole groups
   const size_t diag = std::min(t * tile, na + nb);
   size_t i, j;
   if constexpr (ARITH) {
@@ -239,11 +282,16 @@ partition_kernel(const K *__restrict__ a, size_t na, const K *__restrict__ b, si
       balanced_path_at<true, K>(ra, na, rb, nb, diag,
                                 ordering::sampled_merge_path<K>(ra, na, rb, nb, diag, m, Cmp{}),
                                 Cmp{}, i, j);
+    else if constexpr (G > 1)
+      balanced_path_at<true, K>(ra, na, rb, nb, diag,
+                                ordering::group_merge_path<G, K>(ra, na, rb, nb, diag, Cmp{}),
+                                Cmp{}, i, j);
     else
       balanced_path<true, K>(ra, na, rb, nb, diag, Cmp{}, i, j);
   }
-  splits[2 * t] = i;
-  splits[2 * t + 1] = j;
+  if (thread % G != 0) return;
+  splits[2 * t] = static_cast<S>(i);
+  splits[2 * t + 1] = static_cast<S>(j);
 }
 
 
@@ -252,8 +300,9 @@ struct TileSmem {
   static constexpr uint32_t TILE = THREADS * ITEMS;
   static constexpr uint32_t CAP = TILE + 2;  // a star can make a tile one item longer
   static constexpr bool PAIRS = !std::is_same<V, NoValue>::value;
+  static_assert(CAP <= 65536, "places in a tile are 16-bit");
   K keys[CAP];
-  typename std::conditional<PAIRS, V, char>::type vals[PAIRS ? CAP : 1];
+  uint16_t src[PAIRS ? CAP : 1];  // compacted outputs: their places in the tile
   uint32_t split_a[THREADS + 1];
   uint32_t split_b[THREADS + 1];
   uint32_t wave_total[WAVES];
@@ -302,10 +351,10 @@ __device__ __forceinline__ void serial_step(const K &ka, const K &kb, bool a_ok,
 
 // Outputs of one partition tile, held in registers until the block's output
 // offset is known.
-template <class K, class VS, int ITEMS, bool PAIRS>
+template <class K, int ITEMS, bool PAIRS>
 struct SubTile {
   K outk[ITEMS];
-  VS outv[PAIRS ? ITEMS : 1];
+  uint32_t src[PAIRS ? (ITEMS + 1) / 2 : 1];  // places in the tile, two per word
   uint32_t mask;   // emitted items of this thread
   uint32_t excl;   // this thread's first output within the sub-tile
   uint32_t count;  // the sub-tile's outputs
@@ -315,7 +364,12 @@ struct SubTile {
 // is staged, partitioned and run through the serial operation in turn, its
 // outputs kept in registers; the block then publishes one count and looks
 // back once for all of them, and stores them in turn. SUB = 2 halves the
-// look-backs at the same LDS footprint (two blocks per CU).
+// look-backs at the same LDS footprint (two blocks per CU). Values are not
+// staged: an output keeps its place in the tile, and the store loop reads its
+// value from there (neighbouring outputs read neighbouring values, and only
+// kept values are read). Staged, they filled the registers that the second
+// sub-tile needs and were read whole: 6 x 10^7 u32 keys + 4-byte values, union
+// 347 -> 309 us, intersection 269 -> 191; u64 keys 456 -> 418, 360 -> 262.
 // Two blocks per CU (4 waves per SIMD): a register budget of 128.
 #ifndef RCCL_SET_WAVES_PER_SIMD
 #define RCCL_SET_WAVES_PER_SIMD 4
@@ -323,14 +377,12 @@ struct SubTile {
 template <class K, class V, class Cmp, int OP, int ITEMS, int SUB, bool ARITH>
 __global__ void __launch_bounds__(THREADS, RCCL_SET_WAVES_PER_SIMD)
 tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restrict__ b,
-            const V *__restrict__ bv, const uint64_t *__restrict__ splits, size_t tiles,
+            const V *__restrict__ bv, const Split<SUB> *__restrict__ splits, size_t tiles,
             size_t lb_tiles, K *__restrict__ out, V *__restrict__ outv, size_t out_cap,
             uint64_t *__restrict__ out_count, uint64_t *desc, uint64_t *gagg, uint64_t *ginc,
             uint64_t *ticket, uint32_t nx, Arith<K> ar, Arith<K> br) {
   using Smem = TileSmem<K, V, ITEMS>;
   constexpr bool PAIRS = Smem::PAIRS;
-  constexpr bool VALS_B = PAIRS && (OP == UNION || OP == SYMMETRIC_DIFFERENCE);
-  using VS = typename std::conditional<PAIRS, V, char>::type;
   __shared__ Smem sm;
   const Cmp less{};
   const uint32_t tid = threadIdx.x;
@@ -348,7 +400,6 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
   // clamped to the tile's last item (striped, so the loads coalesce).
   constexpr int STAGE = (Smem::CAP + THREADS - 1) / THREADS;
   K kr[STAGE];
-  VS vr[PAIRS ? STAGE : 1];
   auto load_tile = [&](size_t pt) {
     const size_t i0 = splits[2 * pt], j0 = splits[2 * pt + 1];
     const uint32_t la = static_cast<uint32_t>(splits[2 * pt + 2] - i0);
@@ -361,20 +412,16 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
         kr[k] = len ? (from_a ? arith_at(ar, i0 + i) : arith_at(br, j0 + (i - la))) : K{};
       else
         kr[k] = len ? *(from_a ? a + i0 + i : b + j0 + (i - la)) : K{};
-      if constexpr (PAIRS) {
-        if constexpr (VALS_B) vr[k] = len ? *(from_a ? av + i0 + i : bv + j0 + (i - la)) : V{};
-        else vr[k] = from_a ? av[i0 + i] : V{};
-      }
     }
   };
   if (t * SUB < tiles) load_tile(t * SUB);
 
   // Barriers order LDS only (lds_barrier): the next sub-tile's loads, issued
   // right after the current one is staged, stay in flight through its merge.
-  SubTile<K, VS, ITEMS, PAIRS> sub[SUB];
+  SubTile<K, ITEMS, PAIRS> sub[SUB];
 #pragma unroll
   for (int s = 0; s < SUB; ++s) {
-    SubTile<K, VS, ITEMS, PAIRS> &r = sub[s];
+    SubTile<K, ITEMS, PAIRS> &r = sub[s];
     const size_t pt = t * SUB + s;
     if (pt >= tiles) {  // uniform: the last look-back tile may be short
       r.mask = 0;
@@ -395,7 +442,6 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
       const uint32_t i = uint32_t(k) * THREADS + tid;
       if (i < len) {
         sm.keys[i] = kr[k];
-        if constexpr (PAIRS) sm.vals[i] = vr[k];
       }
     }
     lds_barrier();
@@ -426,7 +472,6 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
     // Serial operation over this thread's A and B ranges.
     uint32_t ia = sm.split_a[tid], ib = sm.split_b[tid];
     const uint32_t ea = max(ia, sm.split_a[tid + 1]), eb = max(ib, sm.split_b[tid + 1]);
-    uint32_t src[PAIRS ? ITEMS : 1];
     uint32_t mask = 0;
     // The heads live in registers; a step reloads only the side it advanced.
     const uint32_t last = len ? len - 1u : 0u;
@@ -438,7 +483,11 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
       bool emit, emit_b, adv_a, adv_b;
       serial_step<OP, K>(ka, kb, a_ok, b_ok, less, emit, emit_b, adv_a, adv_b);
       r.outk[k] = emit_b ? kb : ka;
-      if constexpr (PAIRS) src[k] = emit_b ? la + ib : ia;
+      if constexpr (PAIRS) {
+        const uint32_t place = emit_b ? la + ib : ia;
+        if (k % 2 == 0) r.src[k / 2] = place;
+        else r.src[k / 2] |= place << 16;
+      }
       mask |= emit ? (1u << k) : 0u;
       ia += adv_a ? 1u : 0u;
       ib += adv_b ? 1u : 0u;
@@ -449,10 +498,6 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
     }
     const uint32_t mine = __popc(mask);
     r.mask = mask;
-    if constexpr (PAIRS) {
-#pragma unroll
-      for (int k = 0; k < ITEMS; ++k) r.outv[k] = sm.vals[min(src[k], last)];
-    }
 
     // Block-wide exclusive scan of the emitted counts.
     const uint32_t inc = wave_inclusive_sum(mine, lane);
@@ -472,13 +517,13 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
 #pragma unroll
   for (int s = 0; s < SUB; ++s) total += sub[s].count;
 
-  auto compact = [&](const SubTile<K, VS, ITEMS, PAIRS> &r) {
+  auto compact = [&](const SubTile<K, ITEMS, PAIRS> &r) {
     uint32_t o = r.excl;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       if (r.mask & (1u << k)) {
         sm.keys[o] = r.outk[k];
-        if constexpr (PAIRS) sm.vals[o] = r.outv[k];
+        if constexpr (PAIRS) sm.src[o] = static_cast<uint16_t>(r.src[k / 2] >> (k % 2 * 16));
         ++o;
       }
     }
@@ -504,7 +549,7 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
   size_t base = sm.tile_offset;
 #pragma unroll
   for (int s = 0; s < SUB; ++s) {
-    const SubTile<K, VS, ITEMS, PAIRS> &r = sub[s];
+    const SubTile<K, ITEMS, PAIRS> &r = sub[s];
     if (base >= out_cap) return;  // uniform: the rest lies past the end
     const uint32_t keep = static_cast<uint32_t>(std::min<size_t>(r.count, out_cap - base));
     if (s > 0) {
@@ -513,12 +558,36 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
       lds_barrier();
     }
     constexpr int STORE = (Smem::CAP + THREADS - 1) / THREADS;
+    if constexpr (PAIRS) {
+      // A batch's values are loaded together (up to 18 registers), then stored
+      // with their keys.
+      constexpr int BATCH = sizeof(V) <= 4 ? 18 : (sizeof(V) <= 8 ? 9 : 4);
+      const size_t pt = t * SUB + s;
+      const size_t i0 = keep ? splits[2 * pt] : 0, j0 = keep ? splits[2 * pt + 1] : 0;
+      const uint32_t la = keep ? static_cast<uint32_t>(splits[2 * pt + 2] - i0) : 0u;
 #pragma unroll
-    for (int k = 0; k < STORE; ++k) {
-      const uint32_t i = uint32_t(k) * THREADS + tid;
-      if (i < keep) {
-        out[base + i] = sm.keys[i];
-        if constexpr (PAIRS) outv[base + i] = sm.vals[i];
+      for (int k0 = 0; k0 < STORE; k0 += BATCH) {
+        if (uint32_t(k0) * THREADS >= keep) break;  // uniform
+        V v[BATCH];
+#pragma unroll
+        for (int k = k0; k < k0 + BATCH && k < STORE; ++k) {
+          const uint32_t p = sm.src[min(uint32_t(k) * THREADS + tid, keep - 1u)];
+          v[k - k0] = *(p < la ? av + i0 + p : bv + j0 + (p - la));
+        }
+#pragma unroll
+        for (int k = k0; k < k0 + BATCH && k < STORE; ++k) {
+          const uint32_t i = uint32_t(k) * THREADS + tid;
+          if (i < keep) {
+            out[base + i] = sm.keys[i];
+            outv[base + i] = v[k - k0];
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < STORE; ++k) {
+        const uint32_t i = uint32_t(k) * THREADS + tid;
+        if (i < keep) out[base + i] = sm.keys[i];
       }
     }
     base += r.count;
@@ -547,29 +616,22 @@ struct SetArgs {
 struct Layout {
   size_t tiles = 0, lb_tiles = 0, groups = 0;  // partition tiles, look-back tiles
   size_t splits = 0, desc = 0, gagg = 0, ginc = 0, ticket = 0, samples = 0, total = 0;
-  bool sampled = false;  // integer keys from SAMPLED_MIN_TILES partition tiles
+  bool sampled = false;  // integer keys, from a number of partition tiles
 };
 
-// The sampled merge-path partition serves inputs of at least this many
-// partition tiles (integer keys; arithmetic ranges compute their items and
-// keep the plain search).
-constexpr size_t SAMPLED_MIN_TILES = 512;
-
-// Workspace layout for partition tiles of ITEMS items per thread. Fewer items
-// give more tiles and no smaller a section, so the layout at min_items_for
-// bounds every operation's.
-template <class K, class V, int ITEMS>
-Layout layout(size_t na, size_t nb) {
+// Workspace layout for partition tiles of ITEMS items per thread, SUB of them
+// per look-back tile, with samples from sampled_min tiles.
+template <class K, int ITEMS, int SUB, class S>
+Layout layout(size_t na, size_t nb, size_t sampled_min) {
   Layout l;
   const size_t total = na + nb;
   constexpr size_t TILE = size_t(THREADS) * ITEMS;
   l.tiles = total ? (total + TILE - 1) / TILE : 1;  // an empty input still reports its count
-  constexpr size_t SUB = sub_tiles_for<K, V>();
   l.lb_tiles = (l.tiles + SUB - 1) / SUB;
   l.groups = (l.lb_tiles + GROUP - 1) / GROUP;
   size_t off = 0;
   l.splits = off;
-  off += align_up((l.tiles + 1) * 2 * sizeof(uint64_t), 256);
+  off += align_up((l.tiles + 1) * 2 * sizeof(S), 256);
   // Descriptors, group words and the ticket: one span (lookback::state_layout).
   const lookback::State st = lookback::state_layout(l.lb_tiles);
   l.desc = off;
@@ -577,8 +639,7 @@ Layout layout(size_t na, size_t nb) {
   l.ginc = off + st.ginc * sizeof(uint64_t);
   l.ticket = off + st.ticket * sizeof(uint64_t);
   off += st.words * sizeof(uint64_t);
-  l.sampled = ordering::sampled_partition_for<K>() && na > 0 && nb > 0 &&
-              l.tiles >= SAMPLED_MIN_TILES;
+  l.sampled = ordering::sampled_partition_for<K>() && na > 0 && nb > 0 && l.tiles >= sampled_min;
   if (l.sampled) {
     off = align_up(off, 256);
     l.samples = off;
@@ -587,18 +648,23 @@ Layout layout(size_t na, size_t nb) {
   l.total = align_up(off, 256);
   return l;
 }
+template <class K, class V, int ITEMS>
+size_t workspace_need(size_t na, size_t nb) {
+  return layout<K, ITEMS, workspace_sub_tiles<V>(), uint64_t>(na, nb, WORKSPACE_SAMPLED_MIN).total;
+}
 
-template <class K, class V, class Cmp, int OP>
-rccl_hip_status run_op(const SetArgs &s) {
-  constexpr int ITEMS = items_for<K, V, OP>();
-  constexpr int SUB = sub_tiles_for<K, V>();
+template <class K, class V, class Cmp, int OP, int ITEMS, int SUB, bool ARITH>
+rccl_hip_status run_shape(const SetArgs &s) {
   constexpr size_t TILE = size_t(THREADS) * ITEMS;
-  const Layout l = layout<K, V, ITEMS>(s.na, s.nb);
-  if (!s.ws || s.ws_bytes < l.total)
-    return set_error(RCCL_HIP_ERROR_WORKSPACE_TOO_SMALL, "set operation workspace", l.total,
+  const Layout l = layout<K, ITEMS, SUB, Split<SUB>>(s.na, s.nb, ordering::PARTITION_SAMPLED_MIN);
+  const size_t need = workspace_need<K, V, workspace_items_for<K, V, OP>()>(s.na, s.nb);
+  if (!s.ws || s.ws_bytes < need)
+    return set_error(RCCL_HIP_ERROR_WORKSPACE_TOO_SMALL, "set operation workspace", need,
                      s.ws_bytes);
+  if (l.total > need)
+    return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "set operation layout", need, l.total);
   unsigned char *ws = static_cast<unsigned char *>(s.ws);
-  uint64_t *splits = reinterpret_cast<uint64_t *>(ws + l.splits);
+  Split<SUB> *splits = reinterpret_cast<Split<SUB> *>(ws + l.splits);
   uint64_t *desc = reinterpret_cast<uint64_t *>(ws + l.desc);
   uint64_t *gagg = reinterpret_cast<uint64_t *>(ws + l.gagg);
   uint64_t *ginc = reinterpret_cast<uint64_t *>(ws + l.ginc);
@@ -608,10 +674,8 @@ rccl_hip_status run_op(const SetArgs &s) {
   uint32_t nx = 1;
   RCCL_HIP_TRY(tile_order(&nx, s.stream));
   RCCL_HIP_TRY(fit_tile_order(
-      s.arith ? reinterpret_cast<const void *>(&tile_kernel<K, V, Cmp, OP, ITEMS, SUB, true>)
-              : reinterpret_cast<const void *>(&tile_kernel<K, V, Cmp, OP, ITEMS, SUB, false>),
-      THREADS, XCD_RUN, &nx));
-  const dim3 pgrid(static_cast<uint32_t>((l.tiles + 1 + 255) / 256));
+      reinterpret_cast<const void *>(&tile_kernel<K, V, Cmp, OP, ITEMS, SUB, ARITH>), THREADS,
+      XCD_RUN, &nx));
   const dim3 tgrid(
       static_cast<uint32_t>(nx == XCDS ? xcd_order_grid(l.lb_tiles, XCD_RUN) : l.lb_tiles));
   const K *a = static_cast<const K *>(s.a);
@@ -620,32 +684,16 @@ rccl_hip_status run_op(const SetArgs &s) {
   const V *bv = static_cast<const V *>(s.bv);
   K *out = static_cast<K *>(s.out);
   V *outv = static_cast<V *>(s.outv);
-  if (s.arith) {
-    if constexpr (std::is_integral<K>::value && std::is_same<V, NoValue>::value) {
-      Arith<K> ar, br;
-      std::memcpy(&ar.start, &s.a_start, sizeof(K));
-      std::memcpy(&ar.step, &s.a_step, sizeof(K));
-      std::memcpy(&br.start, &s.b_start, sizeof(K));
-      std::memcpy(&br.step, &s.b_step, sizeof(K));
-      {
-        KernelTimer t("set_partition", s.stream, l.tiles + 1);
-        partition_kernel<K, Cmp, true, false><<<pgrid, 256, 0, s.stream>>>(
-            a, s.na, b, s.nb, TILE, l.tiles + 1, splits, ar, br, desc, state_words, nullptr);
-      }
-      RCCL_HIP_TRY(check_launch("set partition"));
-      {
-        KernelTimer t("set_tile", s.stream, s.na + s.nb);
-        tile_kernel<K, V, Cmp, OP, ITEMS, SUB, true><<<tgrid, THREADS, 0, s.stream>>>(
-            a, av, b, bv, splits, l.tiles, l.lb_tiles, out, outv, s.out_cap, s.out_count, desc, gagg, ginc,
-            ticket, nx, ar, br);
-      }
-      return check_launch("set tile");
-    } else {
-      return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "arithmetic range key kind");
-    }
+  Arith<K> ar{}, br{};
+  if constexpr (ARITH) {
+    std::memcpy(&ar.start, &s.a_start, sizeof(K));
+    std::memcpy(&ar.step, &s.a_step, sizeof(K));
+    std::memcpy(&br.start, &s.b_start, sizeof(K));
+    std::memcpy(&br.step, &s.b_step, sizeof(K));
   }
-  uint32_t *m = l.sampled ? reinterpret_cast<uint32_t *>(ws + l.samples) : nullptr;
-  if (l.sampled) {
+  const bool sampled = !ARITH && l.sampled;
+  uint32_t *m = sampled ? reinterpret_cast<uint32_t *>(ws + l.samples) : nullptr;
+  if (sampled) {
     const size_t ka = ordering::merge_samples(s.na);
     {
       KernelTimer t("set_sample", s.stream, ka);
@@ -657,24 +705,45 @@ rccl_hip_status run_op(const SetArgs &s) {
   }
   {
     KernelTimer t("set_partition", s.stream, l.tiles + 1);
-    if (l.sampled) {
-      partition_kernel<K, Cmp, false, true><<<pgrid, 256, 0, s.stream>>>(
-          a, s.na, b, s.nb, TILE, l.tiles + 1, splits, Arith<K>{}, Arith<K>{}, desc, state_words,
-          m);
-    } else {
-      partition_kernel<K, Cmp, false, false><<<pgrid, 256, 0, s.stream>>>(
-          a, s.na, b, s.nb, TILE, l.tiles + 1, splits, Arith<K>{}, Arith<K>{}, desc, state_words,
-          nullptr);
-    }
+    const auto partition = [&](auto from_samples, auto lanes) {
+      constexpr uint32_t G = decltype(lanes)::value;
+      partition_kernel<K, Cmp, Split<SUB>, ARITH, decltype(from_samples)::value, G>
+          <<<dim3(static_cast<uint32_t>(((l.tiles + 1) * G + 255) / 256)), 256, 0, s.stream>>>(
+              a, s.na, b, s.nb, TILE, l.tiles + 1, splits, ar, br, desc, state_words, m);
+    };
+    using One = std::integral_constant<uint32_t, 1>;
+    if constexpr (ARITH)
+      partition(std::false_type{}, One{});
+    else if (sampled)
+      partition(std::true_type{}, One{});
+    else
+      ordering::with_partition_lanes<K>(
+          l.tiles, [&](auto lanes) { partition(std::false_type{}, lanes); });
   }
   RCCL_HIP_TRY(check_launch("set partition"));
   {
     KernelTimer t("set_tile", s.stream, s.na + s.nb);
-    tile_kernel<K, V, Cmp, OP, ITEMS, SUB, false><<<tgrid, THREADS, 0, s.stream>>>(
-        a, av, b, bv, splits, l.tiles, l.lb_tiles, out, outv, s.out_cap, s.out_count, desc, gagg, ginc,
-        ticket, nx, Arith<K>{}, Arith<K>{});
+    tile_kernel<K, V, Cmp, OP, ITEMS, SUB, ARITH><<<tgrid, THREADS, 0, s.stream>>>(
+        a, av, b, bv, splits, l.tiles, l.lb_tiles, out, outv, s.out_cap, s.out_count, desc, gagg,
+        ginc, ticket, nx, ar, br);
   }
   return check_launch("set tile");
+}
+
+template <class K, class V, class Cmp, int OP, int ITEMS, int SUB>
+rccl_hip_status run_inputs(const SetArgs &s) {
+  if (!s.arith) return run_shape<K, V, Cmp, OP, ITEMS, SUB, false>(s);
+  if constexpr (std::is_integral<K>::value && std::is_same<V, NoValue>::value)
+    return run_shape<K, V, Cmp, OP, ITEMS, SUB, true>(s);
+  else
+    return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "arithmetic range key kind");
+}
+
+template <class K, class V, class Cmp, int OP>
+rccl_hip_status run_op(const SetArgs &s) {
+  if (small_shape<K, V>(s.na + s.nb))
+    return run_inputs<K, V, Cmp, OP, small_items_for<K, V>(), 1>(s);
+  return run_inputs<K, V, Cmp, OP, items_for<K, V, OP>(), SUB_TILES>(s);
 }
 
 template <class K, bool DESC>
@@ -694,7 +763,9 @@ struct KindRunner {
 // Workspace bytes for keys K and values V, whatever the operation.
 template <class K, class V>
 size_t bytes_v(size_t na, size_t nb) {
-  return layout<K, V, min_items_for<K, V>()>(na, nb).total;
+  constexpr int ITEMS = std::min(workspace_items_for<K, V, UNION>(),
+                                 workspace_items_for<K, V, INTERSECTION>());
+  return workspace_need<K, V, ITEMS>(na, nb);
 }
 
 #define RCCL_SET_DECLARE_KIND(NAME)                                                       \

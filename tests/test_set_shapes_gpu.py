@@ -1,0 +1,107 @@
+"""Set operations and merges at the edges of their tile shapes and partitions:
+one or two partition tiles per block, a wave / 16 / 8 lanes per tile boundary,
+against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from rccl_amd import cub, workloads
+from rccl_amd.device import DeviceBuffer
+
+pytestmark = pytest.mark.gpu
+OPS = ("union", "intersection", "difference", "symmetric_difference")
+
+
+def _multiset(dtype, n, seed):
+    """Sorted, about a third of the keys in runs; the type's extremes occur."""
+    dt = np.dtype(dtype)
+    span = np.uint64(max(4, n + n // 2))
+    k = (workloads.hash_range(seed, n) % span).astype(np.uint64)
+    if dt.itemsize == 8:
+        k = k << np.uint64(30)
+    k = k.astype(f"u{dt.itemsize}")
+    k[: n // 50] = 0
+    k[n - n // 40:] = np.iinfo(k.dtype).max
+    return np.sort(k.view(dt))
+
+
+def _same(a, b):
+    return np.array_equal(np.ascontiguousarray(a).view(np.uint8),
+                          np.ascontiguousarray(b).view(np.uint8))
+
+
+# (kind, value bytes, items of a small tile's block, small tiles at most)
+SHAPES = [("u32", 0, 16, 640), ("u32", 4, 16, 640), ("i32", 16, 16, 640), ("u64", 0, 16, 448),
+          ("i64", 8, 14, 448), ("u64", 16, 14, 448)]
+
+
+@pytest.mark.parametrize("kind,width,items,most", SHAPES)
+@pytest.mark.parametrize("where", ["one_tile", "two_tiles", "small_max", "large_min"])
+def test_set_tile_shapes(launch, tile_order, kind, width, items, most, where):
+    tile = 512 * items
+    total = {"one_tile": tile, "two_tiles": tile + 1, "small_max": most * tile,
+             "large_min": most * tile + 1}[where]
+    dt = np.dtype(oracle.KIND_DTYPES[kind])
+    na = total * 2 // 5
+    a, b = _multiset(dt, na, 3 + total), _multiset(dt, total - na, 5 + total)
+    va = vb = None
+    if width:
+        va = workloads.hash_range(11, total * 2)[: na * 2].view(np.uint8)[: na * width]
+        vb = workloads.hash_range(13, total * 2).view(np.uint8)[: (total - na) * width]
+        vt = np.dtype((np.void, 16)) if width == 16 else np.dtype(f"u{width}")
+        va, vb = va.view(vt), vb.view(vt)
+    da, db = DeviceBuffer.from_host(a), DeviceBuffer.from_host(b)
+    dva, dvb = (DeviceBuffer.from_host(va), DeviceBuffer.from_host(vb)) if width else (None, None)
+    for op in OPS:
+        cap = cub.set_output_capacity(op, na, total - na)
+        out = DeviceBuffer.zeroed(dt, cap)
+        if width:
+            outv = DeviceBuffer.zeroed(va.dtype, cap)
+            ws = cub.device_set_pairs_workspace(launch, op, dt, va.dtype, na, total - na)
+            cub.device_set_pairs(launch, op, da, dva, db, dvb, ws, out, outv)
+            wk, wv = oracle.set_op(op, kind, a, b, va, vb)
+        else:
+            ws = cub.device_set_workspace(launch, op, dt, na, total - na)
+            cub.device_set_keys(launch, op, da, db, ws, out)
+            wk = oracle.set_op(op, kind, a, b)
+        m = ws.count()
+        assert m == wk.size, op
+        assert _same(out.to_host_vec()[:m], wk), op
+        if width:
+            assert _same(outv.to_host_vec()[:m], wv), op
+
+
+# Tiles of 2,048 (u32 pairs), 1,536 (16-byte pairs) and 3,072 / 4,096 keys: 255,
+# 256, 2,047, 2,048, 16,383 and 16,384 of them.
+@pytest.mark.parametrize("kind,width,tile", [("u32", 4, 2048), ("u64", 8, 1536), ("i32", 0, 3072)])
+@pytest.mark.parametrize("tiles", [255, 256, 2_047, 2_048, 16_383, 16_384])
+@pytest.mark.parametrize("descending", [False, True])
+def test_merge_partition_lanes(launch, kind, width, tile, tiles, descending):
+    total = tile * tiles
+    if width == 0 and tiles > 2_048:
+        total = 4096 * tiles  # the longer tiles of more than 2^24 keys
+    if descending and tiles > 2_048:
+        pytest.skip("the largest sizes run in one order")
+    na = total // 3
+    dt = np.dtype(oracle.KIND_DTYPES[kind])
+    a, b = _multiset(dt, na, 17 + tiles), _multiset(dt, total - na, 19 + tiles)
+    if descending:
+        a, b = a[::-1].copy(), b[::-1].copy()
+    order = cub.descending if descending else cub.ascending
+    da, db, out = DeviceBuffer.from_host(a), DeviceBuffer.from_host(b), DeviceBuffer.zeroed(dt, total)
+    if width:
+        vt = np.dtype(f"u{width}")
+        va, vb = np.arange(na, dtype=vt), np.arange(na, total, dtype=vt)
+        outv = DeviceBuffer.zeroed(vt, total)
+        ws = cub.device_merge_pairs_workspace(launch, dt, vt, na, total - na)
+        cub.device_merge_pairs(launch, da, DeviceBuffer.from_host(va), db,
+                               DeviceBuffer.from_host(vb), ws, out, outv, order)
+        launch.synchronize()
+        wk, wv = oracle.merge(kind, a, b, va, vb, descending=descending)
+        assert _same(outv.to_host_vec(), wv)
+    else:
+        ws = cub.device_merge_workspace(launch, dt, na, total - na)
+        cub.device_merge_keys(launch, da, db, ws, out, order)
+        launch.synchronize()
+        wk = oracle.merge(kind, a, b, descending=descending)
+    assert _same(out.to_host_vec(), wk)
