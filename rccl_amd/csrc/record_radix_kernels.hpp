@@ -18,9 +18,12 @@
 //               number of active passes, an out-of-place one at least one: a
 //               trivial pass is activated when needed, and is then a stable
 //               copy)
-//   onesweep    one launch per byte position; inactive passes return at once,
-//               active ones run the scalar sort's onesweep tile with rows as
-//               keys (radix_kernels.hpp)
+//   onesweep    launch k runs the k-th active pass: the scalar sort's onesweep
+//               tile with rows as keys (radix_kernels.hpp); a launch past the
+//               last active pass returns at once
+//   tail        the first 2N active passes have launches of their own; one
+//               launch runs all that remain (usually none: rows of interned
+//               ids leave half the byte positions constant)
 #pragma once
 
 #include "radix_kernels.hpp"
@@ -35,16 +38,18 @@ using radix::LookbackBuf;
 // Source/destination buffers: 0 the input, 1 the output, 2 the scratch.
 using radix::PassPlan;
 
-// Onesweep policy for rows: 512 threads x 4 rows = 2048-row tiles for every
-// arity (at most 48 KB of staged rows, two blocks per CU). At the reference
-// workload's 2^20 rows this measured best among 1024- to 4096-row tiles:
-// larger tiles leave CUs idle, smaller ones lengthen the look-back.
+// Onesweep policy for rows: 512 threads, 8 rows each where two staged tiles
+// fit a CU's LDS (6 for 20-byte rows, 5 for 24-byte ones), 4 below
+// LARGE_TILE_MIN_ROWS rows, where large tiles leave CUs idle. Arity 4 with 8-byte
+// payloads, 4 / 8 rows per thread: 2^23 rows 784.6 / 686.6 us, 2^20 160.9 /
+// 155.0; 2 x 10^5 rows without payload 104.0 / 106.4.
 #ifndef RCCL_RECORD_RADIX_THREADS
 #define RCCL_RECORD_RADIX_THREADS 512
 #endif
 #ifndef RCCL_RECORD_RADIX_ITEMS
-#define RCCL_RECORD_RADIX_ITEMS 4
+#define RCCL_RECORD_RADIX_ITEMS 8
 #endif
+constexpr size_t LARGE_TILE_MIN_ROWS = size_t(1) << 19;
 // Below this many rows the merge sort (fewer launches) is used.
 #ifndef RCCL_RECORD_RADIX_MIN_ROWS
 #define RCCL_RECORD_RADIX_MIN_ROWS 65536
@@ -54,17 +59,24 @@ constexpr size_t RADIX_MIN_ROWS = RCCL_RECORD_RADIX_MIN_ROWS;
 // Look-back counts are 30-bit; larger inputs take the merge sort.
 constexpr size_t RADIX_MAX_ROWS = (size_t(1) << 30) - 1;
 
-template <int N, class Val>
+// Rows per thread of the large and the small tile.
+template <int N, class Val, bool LARGE>
 constexpr int radix_items() {
   constexpr size_t vb = std::is_same<Val, radix::NoValue>::value ? 0 : sizeof(Val);
   constexpr size_t elem = 4 * N > vb ? 4 * N : vb;
-  static_assert(size_t(RADIX_THREADS) * RCCL_RECORD_RADIX_ITEMS * elem <= 64 * 1024,
-                "the staged tile must leave room for two blocks per CU");
-  return RCCL_RECORD_RADIX_ITEMS;
+  constexpr size_t fit = 64 * 1024 / (size_t(RADIX_THREADS) * elem);
+  return LARGE ? int(fit < RCCL_RECORD_RADIX_ITEMS ? fit : RCCL_RECORD_RADIX_ITEMS) : 4;
 }
+constexpr bool large_tiles(size_t n) { return n >= LARGE_TILE_MIN_ROWS; }
+
+// Active passes with a launch of their own (the tail runs the rest).
+constexpr uint32_t own_launches(int n) { return 2u * uint32_t(n); }
+// Words after the bins: the histogram's completion count, the tail's ticket
+// and its finished tiles per pass.
+constexpr uint32_t sync_words(int n) { return 2u + 4u * uint32_t(n); }
 
 // ---------------------------------------------------------------------------
-// init: zero the bins and the histogram's completion counter.
+// init: zero the bins and the words after them (sync_words).
 // ---------------------------------------------------------------------------
 namespace {
 __global__ void __launch_bounds__(256) record_init_kernel(uint32_t *words, uint32_t count) {
@@ -79,16 +91,22 @@ __global__ void __launch_bounds__(256) record_init_kernel(uint32_t *words, uint3
 // ---------------------------------------------------------------------------
 constexpr int HIST_THREADS = 1024;
 constexpr int HIST_ITEMS = 4;
+#ifndef RCCL_RECORD_HIST_COPIES
+#define RCCL_RECORD_HIST_COPIES 4
+#endif
+constexpr int HIST_COPIES = RCCL_RECORD_HIST_COPIES;
 static_assert(HIST_THREADS >= BINS, "the plan uses one thread per digit");
 
-// Turns the bins into exclusive offsets and writes the pass plan. Called by
-// every thread of one block; threads past BINS only join the barriers.
+// Turns the bins into exclusive offsets and writes the pass plan, the active
+// passes first: entry k's `active` is 1 + the byte position of the k-th active
+// pass, 0 past the last. Called by every thread of one block.
 template <int N>
 __device__ __forceinline__ void write_plan(uint32_t *__restrict__ bins, uint32_t n,
                                            PassPlan *__restrict__ plan, uint32_t plan_flags) {
   constexpr int P = 4 * N;
   __shared__ uint32_t s_wave[P][BINS / 64];
   __shared__ uint32_t s_trivial[P];
+  __shared__ PassPlan s_plan[P];
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   const bool digit_thread = tid < BINS;
@@ -108,17 +126,31 @@ __device__ __forceinline__ void write_plan(uint32_t *__restrict__ bins, uint32_t
     }
   }
   __syncthreads();
-  if (!digit_thread) return;
+  if (digit_thread) {
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    uint32_t excl = inc[p] - c[p];
-    for (uint32_t w = 0; w < (tid >> 6); ++w) excl += s_wave[p][w];
-    bins[p * BINS + tid] = excl;
+    for (int p = 0; p < P; ++p) {
+      uint32_t excl = inc[p] - c[p];
+      for (uint32_t w = 0; w < (tid >> 6); ++w) excl += s_wave[p][w];
+      bins[p * BINS + tid] = excl;
+    }
   }
-  if (tid != 0) return;
-  uint32_t trivial = 0;
-  for (int p = 0; p < P; ++p) trivial |= s_trivial[p] ? (1u << p) : 0u;
-  radix::assign_plan(P, trivial, plan_flags, plan);
+  if (tid == 0) {
+    uint32_t trivial = 0;
+    for (int p = 0; p < P; ++p) trivial |= s_trivial[p] ? (1u << p) : 0u;
+    radix::assign_plan(P, trivial, plan_flags, s_plan);
+  }
+  __syncthreads();
+  if (tid >= P) return;
+  uint32_t before = 0, active = 0;  // active passes before this one, and all
+  for (int p = 0; p < P; ++p) {
+    const uint32_t on = s_plan[p].active != 0 ? 1u : 0u;
+    before += uint32_t(p) < tid ? on : 0u;
+    active += on;
+  }
+  PassPlan e = s_plan[tid];
+  const uint32_t at = e.active ? before : active + tid - before;
+  e.active = e.active ? tid + 1u : 0u;
+  plan[at] = e;
 }
 
 // Adds one wave's digits of byte `byte` of a column word to the LDS
@@ -144,11 +176,13 @@ row_histogram_kernel(const Row<N> *__restrict__ rows, size_t n, uint32_t *__rest
                      uint32_t *__restrict__ done, PassPlan *__restrict__ plan, uint32_t plan_flags,
                      uint32_t *__restrict__ zero_words, size_t zero_count) {
   constexpr int P = 4 * N;
-  __shared__ uint32_t hist[P * BINS];  // [pass][digit], pass 0 = last column's low byte
+  // [copy][pass][digit], pass 0 = last column's low byte; lane l counts in copy
+  // l % HIST_COPIES (few distinct digits otherwise meet on few counters).
+  __shared__ uint32_t hist[HIST_COPIES * P * BINS];
   __shared__ uint32_t s_last;
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
-  for (uint32_t i = tid; i < P * BINS; i += HIST_THREADS) hist[i] = 0;
+  for (uint32_t i = tid; i < HIST_COPIES * P * BINS; i += HIST_THREADS) hist[i] = 0;
   for (size_t i = size_t(blockIdx.x) * HIST_THREADS + tid; i < zero_count;
        i += size_t(gridDim.x) * HIST_THREADS)
     zero_words[i] = 0;
@@ -172,7 +206,7 @@ row_histogram_kernel(const Row<N> *__restrict__ rows, size_t n, uint32_t *__rest
         const uint32_t w = r[j].w[c];
         const uint32_t w0 = __builtin_amdgcn_readfirstlane(w);
         const uint32_t x = w ^ w0;
-        uint32_t *h = &hist[(N - 1 - c) * 4 * BINS];
+        uint32_t *h = &hist[(lane % HIST_COPIES * P + (N - 1 - c) * 4) * BINS];
 #pragma unroll
         for (int b = 0; b < 4; ++b) count_byte(h + b * BINS, w, w0, x, b, leader, cnt);
       }
@@ -180,7 +214,9 @@ row_histogram_kernel(const Row<N> *__restrict__ rows, size_t n, uint32_t *__rest
   }
   __syncthreads();
   for (uint32_t i = tid; i < P * BINS; i += HIST_THREADS) {
-    const uint32_t v = hist[i];
+    uint32_t v = 0;
+#pragma unroll
+    for (int k = 0; k < HIST_COPIES; ++k) v += hist[k * P * BINS + i];
     if (v) add_agent(&bins[i], v);
   }
   // Completion count. The barrier waits for the block's additions; the count
@@ -208,21 +244,74 @@ struct RowBuffers {
   Val *vout, *vscratch;
 };
 
+// One tile of the active pass `pl`.
 template <int N, class Val, int ITEMS, radix::Rank RANK>
-__global__ void __launch_bounds__(RADIX_THREADS, RCCL_RADIX_WAVES_PER_SIMD)
-row_onesweep_kernel(RowBuffers<N, Val> b, size_t n, uint32_t num_tiles,
-                    const uint32_t *__restrict__ pass_bins, const PassPlan *__restrict__ plan,
-                    LookbackBuf<uint32_t> lb0, LookbackBuf<uint32_t> lb1, uint32_t nx,
-                    uint32_t bit) {
-  const PassPlan pl = *plan;
-  if (!pl.active) return;
+__device__ __forceinline__ void row_pass_tile(RowBuffers<N, Val> b, PassPlan pl,
+                                              size_t n, uint32_t num_tiles,
+                                              const uint32_t *__restrict__ bins,
+                                              LookbackBuf<uint32_t> lb0,
+                                              LookbackBuf<uint32_t> lb1, uint32_t nx,
+                                              uint32_t given_tile) {
+  const uint32_t p = pl.active - 1u;
+  const uint32_t bit = 32u * (uint32_t(N) - 1u - p / 4u) + 8u * (p % 4u);
   const Row<N> *kin = pl.src == 0 ? b.in : (pl.src == 1 ? b.out : b.scratch);
   Row<N> *kout = pl.dst == 1 ? b.out : b.scratch;
   const Val *vin = pl.src == 0 ? b.vin : (pl.src == 1 ? b.vout : b.vscratch);
   Val *vout = pl.dst == 1 ? b.vout : b.vscratch;
   radix::onesweep_tile<Row<N>, Val, RowDigits<N>, ITEMS, uint32_t, RADIX_THREADS, RANK>(
-      kin, kout, vin, vout, n, num_tiles, pass_bins, nullptr, pl.lb ? lb1 : lb0,
-      pl.lb ? lb0 : lb1, nx, bit, 0xFFu, pl.conv);
+      kin, kout, vin, vout, n, num_tiles, bins + size_t(p) * BINS, nullptr, pl.lb ? lb1 : lb0,
+      pl.lb ? lb0 : lb1, nx, bit, 0xFFu, pl.conv, given_tile);
+}
+
+template <int N, class Val, int ITEMS, radix::Rank RANK>
+__global__ void __launch_bounds__(RADIX_THREADS, RCCL_RADIX_WAVES_PER_SIMD)
+row_onesweep_kernel(RowBuffers<N, Val> b, size_t n, uint32_t num_tiles,
+                    const uint32_t *__restrict__ bins, const PassPlan *__restrict__ plan,
+                    LookbackBuf<uint32_t> lb0, LookbackBuf<uint32_t> lb1, uint32_t nx) {
+  const PassPlan pl = *plan;
+  if (!pl.active) return;
+  row_pass_tile<N, Val, ITEMS, RANK>(b, pl, n, num_tiles, bins, lb0, lb1, nx, radix::NO_TILE);
+}
+
+// The active passes from plan entry `first` on, in one launch. A launch that
+// finds nothing to do costs about 4 us, and byte positions that do not vary
+// are most of a relation's; this one replaces the last 2N of them.
+// Blocks claim (pass, tile) tickets in order, so a block that waits, for an
+// earlier tile's look-back or for the previous pass to finish, waits on
+// started blocks only, however many of them are resident. A pass starts when
+// every tile of the one before has been written: each tile's stores are
+// released to the device before it is counted (state[1 + pass]), and the
+// waiting block acquires after the count is complete.
+template <int N, class Val, int ITEMS, radix::Rank RANK>
+__global__ void __launch_bounds__(RADIX_THREADS, RCCL_RADIX_WAVES_PER_SIMD)
+row_tail_kernel(RowBuffers<N, Val> b, size_t n, uint32_t num_tiles,
+                const uint32_t *__restrict__ bins, const PassPlan *__restrict__ plan,
+                LookbackBuf<uint32_t> lb0, LookbackBuf<uint32_t> lb1, uint32_t first,
+                uint32_t *state) {
+  constexpr uint32_t P = 4 * N;
+  if (!plan[first].active) return;
+  __shared__ uint32_t s_ticket;
+  while (true) {
+    __syncthreads();  // the last tile's shared memory is no longer read
+    if (threadIdx.x == 0) s_ticket = add_agent(&state[0], 1u);
+    __syncthreads();
+    const uint32_t ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+    const uint32_t k = ticket / num_tiles;
+    if (first + k >= P) return;
+    const PassPlan pl = plan[first + k];
+    if (!pl.active) return;
+    if (k > 0) {
+      if (threadIdx.x == 0)
+        while (load_agent(&state[k]) != num_tiles) __builtin_amdgcn_s_sleep(2);
+      __syncthreads();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    row_pass_tile<N, Val, ITEMS, RANK>(b, pl, n, num_tiles, bins, lb0, lb1, 1u,
+                                       ticket % num_tiles);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    if (threadIdx.x == 0) add_agent(&state[1 + k], 1u);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -240,14 +329,15 @@ struct RadixLayout {
 template <int N, class Val>
 RadixLayout radix_layout(size_t n) {
   constexpr size_t VB = std::is_same<Val, radix::NoValue>::value ? 0 : sizeof(Val);
-  constexpr size_t TILE = size_t(RADIX_THREADS) * radix_items<N, Val>();
+  const size_t TILE = size_t(RADIX_THREADS) *
+                      (large_tiles(n) ? radix_items<N, Val, true>() : radix_items<N, Val, false>());
   constexpr size_t P = 4 * N;
   RadixLayout l;
   l.tiles = (n + TILE - 1) / TILE;
   l.groups = (l.tiles + radix::GROUP - 1) / radix::GROUP;
   size_t off = 0;
   l.bins = off;
-  off += align_up((P * BINS + 1) * sizeof(uint32_t), 256);  // bins, completion count
+  off += align_up((P * BINS + sync_words(N)) * sizeof(uint32_t), 256);
   l.plan = off;
   off += align_up(P * sizeof(PassPlan), 256);
   l.lb_ginc = align_up(l.tiles * BINS * sizeof(uint32_t), 256);
@@ -275,13 +365,13 @@ struct RecordArgs {
   hipStream_t stream;
 };
 
-// The 4N onesweep launches of a row sort, in one ranking mode.
-template <int N, class Val, radix::Rank RANK>
+// The onesweep launches of a row sort, in one ranking mode and tile shape.
+template <int N, class Val, radix::Rank RANK, bool LARGE>
 rccl_hip_status launch_row_onesweeps(const RecordArgs &a, const RadixLayout &l,
-                                     const RowBuffers<N, Val> &b, const uint32_t *bins,
+                                     const RowBuffers<N, Val> &b, uint32_t *bins,
                                      const PassPlan *plan, const LookbackBuf<uint32_t> (&lb)[2],
                                      uint32_t nx) {
-  constexpr int ITEMS = radix_items<N, Val>();
+  constexpr int ITEMS = radix_items<N, Val, LARGE>();
   constexpr uint32_t P = 4 * N;
   size_t resident = 0;
   RCCL_HIP_TRY(resident_blocks(
@@ -290,17 +380,22 @@ rccl_hip_status launch_row_onesweeps(const RecordArgs &a, const RadixLayout &l,
   // The XCD order needs two rows of runs resident at once; with fewer, blocks
   // claim ticketed tiles instead.
   if (nx == XCDS && resident < 2 * size_t(XCDS) * radix::XCD_RUN) nx = 1;
+  const uint32_t tiles = static_cast<uint32_t>(l.tiles);
   const uint32_t grid = static_cast<uint32_t>(radix::onesweep_grid(l.tiles, nx));
-  for (uint32_t p = 0; p < P; ++p) {
-    const uint32_t word = uint32_t(N) - 1u - p / 4u;
-    const uint32_t bit = 32u * word + 8u * (p % 4u);
+  for (uint32_t k = 0; k < own_launches(N); ++k) {
     KernelTimer t("record_onesweep", a.stream, a.n);
     row_onesweep_kernel<N, Val, ITEMS, RANK><<<dim3(grid), RADIX_THREADS, 0, a.stream>>>(
-        b, a.n, static_cast<uint32_t>(l.tiles), bins + size_t(p) * BINS, plan + p, lb[0], lb[1],
-        nx, bit);
+        b, a.n, tiles, bins, plan + k, lb[0], lb[1], nx);
     RCCL_HIP_TRY(check_launch("record sort onesweep"));
   }
-  return ok();
+  {
+    KernelTimer t("record_tail", a.stream, a.n);
+    const size_t blocks = std::min<size_t>(l.tiles, std::max<size_t>(resident, 1));
+    row_tail_kernel<N, Val, ITEMS, RANK>
+        <<<dim3(static_cast<uint32_t>(blocks)), RADIX_THREADS, 0, a.stream>>>(
+            b, a.n, tiles, bins, plan, lb[0], lb[1], own_launches(N), bins + P * BINS + 1);
+  }
+  return check_launch("record sort tail");
 }
 
 template <int N, class Val>
@@ -335,7 +430,7 @@ rccl_hip_status run_radix(const RecordArgs &a) {
 
   {
     KernelTimer t("record_init", a.stream, 0);
-    record_init_kernel<<<1, 256, 0, a.stream>>>(bins, P * BINS + 1);
+    record_init_kernel<<<1, 256, 0, a.stream>>>(bins, P * BINS + sync_words(N));
   }
   RCCL_HIP_TRY(check_launch("record sort init"));
   {
@@ -355,11 +450,14 @@ rccl_hip_status run_radix(const RecordArgs &a) {
         l.lb_bytes / sizeof(uint32_t));
   }
   RCCL_HIP_TRY(check_launch("record sort histogram"));
-  return caps.rank == radix::Rank::LaneAtomic
-             ? launch_row_onesweeps<N, Val, radix::Rank::LaneAtomic>(a, l, b, bins, plan, lb,
-                                                                     caps.nx)
-             : launch_row_onesweeps<N, Val, radix::Rank::MatchAny>(a, l, b, bins, plan, lb,
-                                                                   caps.nx);
+  constexpr radix::Rank LA = radix::Rank::LaneAtomic, MA = radix::Rank::MatchAny;
+  if (large_tiles(a.n))
+    return caps.rank == LA
+               ? launch_row_onesweeps<N, Val, LA, true>(a, l, b, bins, plan, lb, caps.nx)
+               : launch_row_onesweeps<N, Val, MA, true>(a, l, b, bins, plan, lb, caps.nx);
+  return caps.rank == LA
+             ? launch_row_onesweeps<N, Val, LA, false>(a, l, b, bins, plan, lb, caps.nx)
+             : launch_row_onesweeps<N, Val, MA, false>(a, l, b, bins, plan, lb, caps.nx);
 }
 
 } // namespace record_sort
