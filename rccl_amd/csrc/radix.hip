@@ -269,8 +269,7 @@ rccl_hip_status sort_buffer(rccl_hip_key_kind key, size_t value_bytes, rccl_hip_
 
 size_t merge_sort_lowering_bytes(size_t key_bytes_, size_t value_bytes, size_t n) {
   return align_up(n * key_bytes_, 256) + align_up(n * value_bytes, 256) +
-         layout(key_bytes_, value_bytes, n, true).total + plan_bytes() +
-         short_sample_bytes(key_bytes_, n);
+         planned_query_bytes(key_bytes_, value_bytes, n);
 }
 
 // A stable LSD radix sort under the natural order or its reverse yields
@@ -292,9 +291,10 @@ rccl_hip_status merge_sort_lowering(rccl_hip_key_kind key, size_t value_bytes, b
       key != RCCL_HIP_KEY_U64 && key != RCCL_HIP_KEY_I64 && key != RCCL_HIP_KEY_F64)
     return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "merge sort radix key kind");
   const size_t scratch = align_up(n * kb, 256) + align_up(n * value_bytes, 256);
-  if (!workspace || workspace_bytes < merge_sort_lowering_bytes(kb, value_bytes, n))
-    return set_error(RCCL_HIP_ERROR_WORKSPACE_TOO_SMALL, "merge sort workspace",
-                     merge_sort_lowering_bytes(kb, value_bytes, n), workspace_bytes);
+  const size_t need = scratch + planned_bytes(kb, value_bytes, n);
+  if (!workspace || workspace_bytes < need)
+    return set_error(RCCL_HIP_ERROR_WORKSPACE_TOO_SMALL, "merge sort workspace", need,
+                     workspace_bytes);
   unsigned char *ws = static_cast<unsigned char *>(workspace);
   SortArgs a{};
   a.keys[0] = out_keys;

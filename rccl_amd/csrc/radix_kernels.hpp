@@ -1195,14 +1195,14 @@ rccl_hip_status run_passes(SortArgs &a, const Layout &l, uint32_t passes) {
   constexpr int SITEMS = small_items_for(sizeof(Bits), VBYTES);
   constexpr Rank LA = Rank::LaneAtomic, MA = Rank::MatchAny;
   const bool la = caps.rank == LA;
-  if (a.planned)
-    return la ? launch_onesweeps<Bits, Val, Ops, Desc, LA, THREADS, ITEMS, true>(
-                    a, l, passes, bins, skew, plan, caps.nx)
-              : launch_onesweeps<Bits, Val, Ops, Desc, MA, THREADS, ITEMS, true>(
-                    a, l, passes, bins, skew, plan, caps.nx);
-  // Small tiles serve unplanned sorts only, all below 2^30 items (32-bit
-  // descriptors); the layout chose them for this n.
+  // Small tiles: far fewer than 2^30 items, so 32-bit descriptors; the layout
+  // chose them for this n.
   if constexpr (sizeof(Desc) == 4) {
+    if (l.small && a.planned)
+      return la ? launch_onesweeps<Bits, Val, Ops, Desc, LA, SMALL_THREADS, SITEMS, true>(
+                      a, l, passes, bins, skew, plan, caps.nx)
+                : launch_onesweeps<Bits, Val, Ops, Desc, MA, SMALL_THREADS, SITEMS, true>(
+                      a, l, passes, bins, skew, plan, caps.nx);
     if (l.small)
       return la ? launch_onesweeps<Bits, Val, Ops, Desc, LA, SMALL_THREADS, SITEMS, false>(
                       a, l, passes, bins, skew, plan, caps.nx)
@@ -1210,6 +1210,11 @@ rccl_hip_status run_passes(SortArgs &a, const Layout &l, uint32_t passes) {
                       a, l, passes, bins, skew, plan, caps.nx);
   }
   if (l.small) return set_error(RCCL_HIP_ERROR_INVALID_ARGUMENT, "radix small-tile layout");
+  if (a.planned)
+    return la ? launch_onesweeps<Bits, Val, Ops, Desc, LA, THREADS, ITEMS, true>(
+                    a, l, passes, bins, skew, plan, caps.nx)
+              : launch_onesweeps<Bits, Val, Ops, Desc, MA, THREADS, ITEMS, true>(
+                    a, l, passes, bins, skew, plan, caps.nx);
   return la ? launch_onesweeps<Bits, Val, Ops, Desc, LA, THREADS, ITEMS, false>(
                   a, l, passes, bins, skew, plan, caps.nx)
             : launch_onesweeps<Bits, Val, Ops, Desc, MA, THREADS, ITEMS, false>(

@@ -107,12 +107,16 @@ constexpr size_t tile_items(size_t key_bytes, size_t value_bytes) {
 // spreads over every CU: 2^20 u32 keys make 241 tiles instead of 61 (76 -> 66
 // us per sort). Measured crossover: small tiles are faster up to 2^21 u32 keys
 // and 2^20 u64 + u32 pairs (512 small tiles), slower from 2^22 and 2^21.
-// Sorts with a pass plan (the merge-sort lowering) keep the large tiles.
+// Sorts with a pass plan (the merge-sort lowering) take them by the same rule:
+// u32 + u32 comparator sorts of 2^18 pairs 82.3 -> 47.4 us, 2^20 96.1 -> 65.8.
 #ifndef RCCL_RADIX_SMALL_THREADS
 #define RCCL_RADIX_SMALL_THREADS 256
 #endif
 #ifndef RCCL_RADIX_SMALL_MAX_TILES
 #define RCCL_RADIX_SMALL_MAX_TILES 512
+#endif
+#ifndef RCCL_RADIX_PLANNED_SMALL_MAX_TILES
+#define RCCL_RADIX_PLANNED_SMALL_MAX_TILES 512
 #endif
 #ifndef RCCL_RADIX_SMALL_ITEMS_DIV
 #define RCCL_RADIX_SMALL_ITEMS_DIV 2
@@ -126,13 +130,6 @@ constexpr int small_items_for(size_t key_bytes, size_t value_bytes) {
 constexpr size_t small_tile_items(size_t key_bytes, size_t value_bytes) {
   return size_t(SMALL_THREADS) * small_items_for(key_bytes, value_bytes);
 }
-// Whether a sort of n items uses the small tiles (the layout and the launches
-// both ask this).
-constexpr bool small_tiles(size_t key_bytes, size_t value_bytes, size_t n, bool planned) {
-  return !planned && n <= size_t(RCCL_RADIX_SMALL_MAX_TILES) * small_tile_items(key_bytes,
-                                                                               value_bytes);
-}
-
 // Short sorts (radix_block_kernels.hpp): one block sorts its tile in LDS, up
 // to 16 such tiles are then merged by rank; one or two launches where the
 // onesweep takes three and one per key byte. A block is as wide as the CU
@@ -176,6 +173,17 @@ constexpr size_t single_tile_items(size_t key_bytes, size_t value_bytes) {
 // Comparator sorts (DeviceMergeSort) of fewer items also run on a device that
 // was not probed, under graph capture too.
 constexpr size_t COMPARATOR_MIN_ITEMS = 65536;
+
+// Whether a sort of n items uses the small tiles (the layout and the launches
+// both ask this). A planned short sort has no onesweep; its layout stays the
+// smaller one of the large tiles.
+constexpr size_t small_tile_max(size_t key_bytes, size_t value_bytes, bool planned) {
+  return size_t(planned ? RCCL_RADIX_PLANNED_SMALL_MAX_TILES : RCCL_RADIX_SMALL_MAX_TILES) *
+         small_tile_items(key_bytes, value_bytes);
+}
+constexpr bool small_tiles(size_t key_bytes, size_t value_bytes, size_t n, bool planned) {
+  return n <= small_tile_max(key_bytes, value_bytes, planned) && !(planned && short_sort(n));
+}
 
 // Pass plan of a sort that skips trivial passes (one digit holds every key:
 // the pass would not move anything). Buffers: 0 the input, 1 the output,
@@ -280,6 +288,24 @@ inline Layout layout(size_t key_bytes, size_t value_bytes, size_t n, bool planne
 // Workspace of a planned sort's pass plan (one PassPlan per pass, at most 8),
 // after the layout's total.
 inline size_t plan_bytes() { return align_up(8 * sizeof(PassPlan), 256); }
+
+// Workspace a planned sort of n items needs after its scratch keys and values:
+// the layout, the plan and a short sort's samples.
+inline size_t planned_bytes(size_t key_bytes, size_t value_bytes, size_t n) {
+  return layout(key_bytes, value_bytes, n, true).total + plan_bytes() +
+         short_sample_bytes(key_bytes, n);
+}
+// What a query for n items reports: also enough for fewer items, whose small
+// tiles and samples can take more control words than n items' large tiles, so
+// that a workspace made for the largest sort serves every shorter one.
+inline size_t planned_query_bytes(size_t key_bytes, size_t value_bytes, size_t n) {
+  const size_t small = small_tile_max(key_bytes, value_bytes, true);
+  const size_t below = n < small ? n : small;
+  const size_t own = layout(key_bytes, value_bytes, n, true).total;
+  const size_t less = layout(key_bytes, value_bytes, below, true).total;
+  return (own > less ? own : less) + plan_bytes() +
+         short_sample_bytes(key_bytes, n < SHORT_ITEMS ? n : SHORT_ITEMS);
+}
 
 } // namespace radix
 } // namespace rccl_hip

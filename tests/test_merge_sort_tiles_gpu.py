@@ -1,0 +1,66 @@
+"""Comparator sorts at the ends of their tile shapes: the first onesweep after
+the short sorts, the last small tile and the first large one; and the size of a
+workspace, which never falls as the items grow."""
+import numpy as np
+import pytest
+
+import oracle
+import radix_shapes
+from rccl_amd import _abi, cub, workloads
+from rccl_amd.device import DeviceBuffer
+
+SHORT_ITEMS = 131_072
+
+
+def _sizes(kb, vb):
+    most = radix_shapes.small_tile_max(kb, vb)
+    return [SHORT_ITEMS + 1, most // 2 + 1, most, most + 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,width", [("u32", 0), ("f32", 4), ("i32", 16), ("u64", 4),
+                                        ("i64", 0), ("f64", 8)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_comparator_tile_shapes(launch, radix_ranking, kind, width, in_place):
+    dt = np.dtype(oracle.KIND_DTYPES[kind])
+    vt = {0: None, 4: np.dtype(np.uint32), 8: np.dtype(np.uint64),
+          16: np.dtype((np.void, 16))}[width]
+    for n in _sizes(dt.itemsize, width):
+        ws = cub.device_merge_sort_pairs_workspace(launch, dt, vt, n) if width else \
+            cub.device_merge_sort_workspace(launch, dt, n)
+        # Ties, and a constant byte: a pass that the plan skips.
+        raw = workloads.hash_range(n, n)
+        host = (raw % np.uint64(60_000)).astype(np.int64).astype(dt)
+        descending = n % 2 == 1
+        order = cub.descending if descending else cub.ascending
+        keys = DeviceBuffer.from_host(host)
+        out = keys if in_place else DeviceBuffer.zeroed(dt, n)
+        if width:
+            vals_h = workloads.hash_range(5, 2 * n).view(vt) if width == 16 else \
+                np.arange(n).astype(vt)
+            vals = DeviceBuffer.from_host(vals_h)
+            outv = vals if in_place else DeviceBuffer.zeroed(vt, n)
+            if in_place:
+                cub.device_merge_sort_pairs(launch, keys, vals, ws, order)
+            else:
+                cub.device_merge_sort_pairs_copy(launch, keys, vals, ws, out, outv, order)
+        elif in_place:
+            cub.device_merge_sort_keys(launch, keys, ws, order)
+        else:
+            cub.device_merge_sort_keys_copy(launch, keys, ws, out, order)
+        launch.synchronize()
+        at = np.argsort(-host.astype(np.int64) if descending else host.astype(np.int64),
+                        kind="stable")
+        assert np.array_equal(out.to_host_vec(), host[at]), n
+        if width:
+            assert outv.to_host_vec().tobytes() == vals_h[at].tobytes(), n
+
+
+@pytest.mark.parametrize("key,kb", [(0, 4), (3, 8)])
+@pytest.mark.parametrize("vb", [0, 4, 8, 16])
+def test_comparator_workspace_serves_fewer_items(key, kb, vb):
+    sizes = sorted({n + d for n in _sizes(kb, vb) + [5_000, 65_536, SHORT_ITEMS, 1 << 22]
+                    for d in (-1, 0, 1)})
+    need = [_abi.workspace_bytes("rccl_hip_merge_sort_workspace_bytes", key, vb, n)
+            for n in sizes]
+    assert need == sorted(need)
