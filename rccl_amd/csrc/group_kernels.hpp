@@ -10,14 +10,21 @@
 // a run's aggregate is a left fold, ((v0 op v1) op v2) ..., in index order.
 // The reference marks run heads, scans them and folds each run on one thread
 // in three launches. Here one pass over the input does all of it:
-//   tile    one block per tile (tiles in XCD order or from a ticket,
-//           lookback::claim_tile): keys
-//           (and values) staged in LDS, run heads per thread, a block scan
-//           of the head counts, the tile's output offset from a two-level
-//           decoupled look-back (tile_lookback.hpp); for a reduction the
-//           thread holding a head folds its run in index order, from LDS and,
-//           past the tile's end, from global memory; results compacted in
-//           LDS and stored coalesced; the last tile writes the count
+//   tile    a block takes one tile, or 4 or 8 of a large input (tiles_per_block;
+//           blocks in XCD order or from a ticket, lookback::claim_tile). Several
+//           tiles' run heads are counted first, from the keys alone, so that the
+//           block's output offset, a two-level decoupled look-back
+//           (tile_lookback.hpp), is there when the first is stored. A tile's
+//           items are staged in LDS and read back as each thread's consecutive
+//           ones; heads, a block scan of their counts, and for a reduction the
+//           fold in registers: only a thread's last run goes on in LDS and, past
+//           the tile's end, in global memory. Results are compacted in LDS and
+//           stored coalesced; the last block writes the count.
+// What bounds it: HBM bytes on large inputs, the look-back's round trips and the
+// clearing launch on small ones. A call on 2^26 u32 keys + u64 values (1.07 GB,
+// and 0.27 GB for the second read of the keys) took 647 us when the thread of
+// every head walked its run in LDS, 560 with the folds in registers and odd
+// strides, and takes 341 with several tiles per block (2^24: 167, 146, 106).
 // Keys compare with ==: scalar keys (floats by IEEE ==, so NaN keys never
 // join a run) or [u32; N] rows (all columns equal). A key may carry a payload
 // that takes no part in the comparison (the reference's key/value ranges
@@ -93,8 +100,13 @@ struct IndependentProbabilityOr {  // f64: l + r - l * r, clamped to [0, 1]
   }
 };
 
+// Items per thread, odd: a thread reads its consecutive items from LDS, and an
+// odd stride of 4- or 8-byte items puts a wave's lanes on different banks.
 #ifndef RCCL_GROUP_ITEMS_8B
-#define RCCL_GROUP_ITEMS_8B 16
+#define RCCL_GROUP_ITEMS_8B 17
+#endif
+#ifndef RCCL_GROUP_ITEMS_16B
+#define RCCL_GROUP_ITEMS_16B 13
 #endif
 constexpr int THREADS = 256;
 constexpr uint32_t XCD_RUN = 8;  // tiles per XCD run (xcd_order_tile)
@@ -107,7 +119,8 @@ constexpr size_t bytes_of() {
 template <class K, class P, class V>
 constexpr int items_for() {
   constexpr size_t bytes = sizeof(K) + bytes_of<P>() + bytes_of<V>();
-  return bytes <= 8 ? RCCL_GROUP_ITEMS_8B : (bytes <= 16 ? 12 : (bytes <= 32 ? 8 : 6));
+  return bytes <= 8 ? RCCL_GROUP_ITEMS_8B
+                    : (bytes <= 16 ? RCCL_GROUP_ITEMS_16B : (bytes <= 32 ? 7 : 5));
 }
 template <class K, class P, class V>
 constexpr size_t tile_items() {
@@ -136,7 +149,7 @@ group_tile_kernel(const K *__restrict__ keys, const P *__restrict__ pays,
                   K *__restrict__ out_keys, P *__restrict__ out_pays,
                   typename Op::Value *__restrict__ out_vals, uint64_t *__restrict__ out_count,
                   uint64_t *desc, uint64_t *gagg, uint64_t *ginc, uint64_t *ticket,
-                  uint32_t nx) {
+                  uint32_t nx, uint32_t subs) {
   using V = typename Op::Value;
   using Smem = TileSmem<K, P, V, ITEMS>;
   constexpr bool HAS_P = Smem::HAS_P;
@@ -152,126 +165,179 @@ group_tile_kernel(const K *__restrict__ keys, const P *__restrict__ pays,
   __shared__ uint64_t s_tile;
   const size_t t = lookback::claim_tile<XCD_RUN>(nx, ticket, s_tile);
   if (t >= tiles) return;
-  const size_t base = t * TILE;
-  const uint32_t len = static_cast<uint32_t>(std::min<size_t>(TILE, n - base));
+  const size_t span = size_t(TILE) * subs;
+  const size_t begin = t * span;
+  const size_t end = std::min<size_t>(n, begin + span);
 
-  // Stage the tile (striped, coalesced; clamped loads) and the key before it.
-  {
-    K kr[ITEMS];
-    Reg<P> pr[HAS_P ? ITEMS : 1];
-    Reg<V> vr[HAS_V ? ITEMS : 1];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const uint32_t i = min(uint32_t(k) * THREADS + tid, len - 1u);
-      assign(kr[k], keys[base + i]);
-      if constexpr (HAS_P) pr[k] = pays[base + i];
-      if constexpr (HAS_V) vr[k] = vals[base + i];
+  // A block of several tiles counts its run heads first, so that its look-back
+  // has run its course when the first of them is ready to be stored.
+  uint32_t count = 0;
+  if (subs > 1) {
+    uint32_t heads = 0;
+#pragma unroll 8
+    for (size_t i = begin + tid; i < end; i += THREADS) {
+      K before, item;
+      assign(item, keys[i]);
+      assign(before, keys[i > 0 ? i - 1 : 0]);
+      heads += (i == 0 || !eq(before, item)) ? 1u : 0u;
     }
-    if (tid == 0 && t > 0) assign(sm.keys[0], keys[base - 1]);
+    heads = wave_inclusive_sum(heads, lane);
+    if (lane == 63) sm.wave_total[wave] = heads;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) count += sm.wave_total[w];
+    if (tid == 0) lookback::tile_publish(t, count, desc, gagg);
+  }
+
+  size_t done = 0;  // outputs of the block's earlier tiles
+  for (size_t base = begin; base < end; base += TILE) {
+    const uint32_t len = static_cast<uint32_t>(std::min<size_t>(TILE, end - base));
+
+    // Stage the tile (striped, coalesced; clamped loads) and the key before it.
+    {
+      K kr[ITEMS];
+      Reg<P> pr[HAS_P ? ITEMS : 1];
+      Reg<V> vr[HAS_V ? ITEMS : 1];
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t i = min(uint32_t(k) * THREADS + tid, len - 1u);
+        assign(kr[k], keys[base + i]);
+        if constexpr (HAS_P) pr[k] = pays[base + i];
+        if constexpr (HAS_V) vr[k] = vals[base + i];
+      }
+      if (tid == 0 && base > 0) assign(sm.keys[0], keys[base - 1]);
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t i = uint32_t(k) * THREADS + tid;
+        if (i < len) {
+          assign(sm.keys[1 + i], kr[k]);
+          if constexpr (HAS_P) sm.pays[i] = pr[k];
+          if constexpr (HAS_V) sm.vals[i] = vr[k];
+        }
+      }
+    }
+    __syncthreads();
+
+    // This thread's ITEMS consecutive items and the run heads among them. (Slots
+    // past the tile's length hold no head, and their values reach no output.)
+    const uint32_t first = tid * uint32_t(ITEMS);
+    K key[ITEMS];
+    Reg<P> pay[HAS_P ? ITEMS : 1];
+    Reg<V> val[HAS_V ? ITEMS : 1];
+    uint32_t mask = 0;
+    {
+      K prev;
+      assign(prev, sm.keys[first]);
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        const uint32_t i = first + uint32_t(k);
+        assign(key[k], sm.keys[1 + i]);
+        if constexpr (HAS_P) pay[k] = sm.pays[i];
+        if constexpr (HAS_V) val[k] = sm.vals[i];
+        const bool head = i < len && ((base + i == 0) || !eq(prev, key[k]));
+        mask |= head ? (1u << k) : 0u;
+        assign(prev, key[k]);
+      }
+    }
+    const uint32_t mine = __popc(mask);
+
+    // Block-wide exclusive scan of the head counts. A single tile's count is
+    // published before the folds, which later tiles' look-backs need not wait for.
+    const uint32_t inc = wave_inclusive_sum(mine, lane);
+    if (lane == 63) sm.wave_total[wave] = inc;
+    __syncthreads();
+    uint32_t excl = inc - mine;
+    uint32_t tile_count = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (uint32_t(w) < wave) excl += sm.wave_total[w];
+      tile_count += sm.wave_total[w];
+    }
+    if (subs == 1) {
+      count = tile_count;
+      if (tid == 0) lookback::tile_publish(t, count, desc, gagg);
+    }
+
+    // Fold in index order, in registers: val[k] becomes its run's fold up to item
+    // k (of use from the thread's first head on). The thread's last run goes on
+    // past its items, in LDS and then in global memory.
+    Reg<V> last{};
+    if constexpr (HAS_V) {
+      const Op op{};
+#pragma unroll
+      for (int k = 1; k < ITEMS; ++k) {
+        if (first + uint32_t(k) < len && !(mask & (1u << k))) val[k] = op(val[k - 1], val[k]);
+        else if (first + uint32_t(k) >= len) val[k] = val[k - 1];
+      }
+      last = val[ITEMS - 1];
+      if (mask != 0) {
+        uint32_t j = first + uint32_t(ITEMS);
+        K prev;
+        assign(prev, key[ITEMS - 1]);
+        bool more = true;
+        while (more && j < len) {
+          K next;
+          assign(next, sm.keys[1 + j]);
+          more = eq(prev, next);
+          if (more) last = op(last, sm.vals[j]);
+          assign(prev, next);
+          ++j;
+        }
+        if (more && j >= len) {
+          size_t g = base + len;
+          if (g < n) assign(prev, sm.keys[len]);
+          while (g < n) {
+            K next;
+            assign(next, keys[g]);
+            if (!eq(prev, next)) break;
+            last = op(last, vals[g]);
+            assign(prev, next);
+            ++g;
+          }
+        }
+      }
+    }
+    __syncthreads();  // the staged tile is no longer read
+
+    // One wave looks back while the others compact through LDS.
+    if (base == begin && wave == 0) {
+      const uint64_t prefix = lookback::tile_resolve(t, tiles, count, desc, gagg, ginc, lane);
+      if (lane == 0) {
+        if (t + 1 == tiles) *out_count = prefix + count;
+        sm.tile_offset = prefix;
+      }
+    }
+    {
+      uint32_t o = excl;
+#pragma unroll
+      for (int k = 0; k < ITEMS; ++k) {
+        if (mask & (1u << k)) {
+          assign(sm.keys[o], key[k]);
+          if constexpr (HAS_P) sm.pays[o] = pay[k];
+          // The run before this one in the thread ends at item k - 1.
+          if constexpr (HAS_V) {
+            if (k > 0 && o > excl) sm.vals[o - 1] = val[k > 0 ? k - 1 : 0];
+          }
+          ++o;
+        }
+      }
+      if constexpr (HAS_V) {
+        if (mine) sm.vals[o - 1] = last;
+      }
+    }
+    __syncthreads();
+    const size_t obase = sm.tile_offset + done;
+    done += tile_count;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const uint32_t i = uint32_t(k) * THREADS + tid;
-      if (i < len) {
-        assign(sm.keys[1 + i], kr[k]);
-        if constexpr (HAS_P) sm.pays[i] = pr[k];
-        if constexpr (HAS_V) sm.vals[i] = vr[k];
+      if (i < tile_count) {
+        assign(out_keys[obase + i], sm.keys[i]);
+        if constexpr (HAS_P) out_pays[obase + i] = sm.pays[i];
+        if constexpr (HAS_V) out_vals[obase + i] = sm.vals[i];
       }
     }
-  }
-  __syncthreads();
-
-  // Run heads among this thread's ITEMS consecutive items.
-  const uint32_t first = tid * uint32_t(ITEMS);
-  uint32_t mask = 0;
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const uint32_t i = first + uint32_t(k);
-    const bool head = i < len && ((base + i == 0) || !eq(sm.keys[i], sm.keys[1 + i]));
-    mask |= head ? (1u << k) : 0u;
-  }
-  const uint32_t mine = __popc(mask);
-
-  // Each head's key and payload; for a reduction, the fold of its run in
-  // index order. A run ends at the next head; past the tile it continues in
-  // global memory.
-  K outk[ITEMS];
-  Reg<P> outp[HAS_P ? ITEMS : 1];
-  Reg<V> outv[HAS_V ? ITEMS : 1];
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    if (!(mask & (1u << k))) continue;
-    const uint32_t i = first + uint32_t(k);
-    assign(outk[k], sm.keys[1 + i]);
-    if constexpr (HAS_P) outp[k] = sm.pays[i];
-    if constexpr (HAS_V) {
-      const Op op{};
-      V agg = sm.vals[i];
-      uint32_t j = i + 1;
-      while (j < len && eq(sm.keys[j], sm.keys[1 + j])) {
-        agg = op(agg, sm.vals[j]);
-        ++j;
-      }
-      if (j == len) {
-        size_t g = base + len;
-        K prev;
-        assign(prev, sm.keys[len]);
-        while (g < n) {
-          K next;
-          assign(next, keys[g]);
-          if (!eq(prev, next)) break;
-          agg = op(agg, vals[g]);
-          assign(prev, next);
-          ++g;
-        }
-      }
-      outv[k] = agg;
-    }
-  }
-
-  // Block-wide exclusive scan of the head counts.
-  const uint32_t inc = wave_inclusive_sum(mine, lane);
-  if (lane == 63) sm.wave_total[wave] = inc;
-  __syncthreads();
-  uint32_t excl = inc - mine;
-  uint32_t tile_count = 0;
-#pragma unroll
-  for (int w = 0; w < WAVES; ++w) {
-    if (uint32_t(w) < wave) excl += sm.wave_total[w];
-    tile_count += sm.wave_total[w];
-  }
-  if (wave == 0) {
-    const uint64_t prefix = lookback::tile_prefix(t, tiles, tile_count, desc, gagg, ginc, lane);
-    if (lane == 0) {
-      if (t + 1 == tiles) *out_count = prefix + tile_count;
-      sm.tile_offset = prefix;
-    }
-  }
-
-  // Compact through LDS (the staged tile is no longer read), then coalesced
-  // stores.
-  __syncthreads();
-  {
-    uint32_t o = excl;
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      if (mask & (1u << k)) {
-        assign(sm.keys[o], outk[k]);
-        if constexpr (HAS_P) sm.pays[o] = outp[k];
-        if constexpr (HAS_V) sm.vals[o] = outv[k];
-        ++o;
-      }
-    }
-  }
-  __syncthreads();
-  const size_t obase = sm.tile_offset;
-#pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const uint32_t i = uint32_t(k) * THREADS + tid;
-    if (i < tile_count) {
-      assign(out_keys[obase + i], sm.keys[i]);
-      if constexpr (HAS_P) out_pays[obase + i] = sm.pays[i];
-      if constexpr (HAS_V) out_vals[obase + i] = sm.vals[i];
-    }
+    __syncthreads();  // before the next tile is staged
   }
 }
 
@@ -295,25 +361,33 @@ struct GroupArgs {
   hipStream_t stream;
 };
 
+// Tiles per block. A block's look-back takes about as long as all else that it
+// does for one tile: at 2^26 u32 + u64 items a reduction's kernel took 518 us,
+// and 205 with the look-back's result made up. Several tiles share one, for a
+// second read of their keys. Kernel us at 1, 2, 4, 8 and 16 tiles per block:
+//   2^22 items (1,261 tiles)    31.0   33.6   31.4   45.1   81.7
+//   2^24       (5,042 tiles)     119   94.3   85.1   98.2   94.3
+//   2^26      (20,165 tiles)     504    373    343    320    356
+// Below 2,048 tiles every block is resident at once, more or less, and fewer
+// blocks would leave CUs idle.
+constexpr size_t ONE_TILE_MAX = 2048, FOUR_TILES_MAX = 8192;
+constexpr uint32_t tiles_per_block(size_t tiles) {
+  return tiles <= ONE_TILE_MAX ? 1u : (tiles <= FOUR_TILES_MAX ? 4u : 8u);
+}
+
 struct Layout {
-  size_t tiles = 0, groups = 0;
-  size_t desc = 0, gagg = 0, ginc = 0, ticket = 0, total = 0;
+  size_t tiles = 0, total = 0;
 };
 
+// Room for the look-back state of one tile per block, the most there can be, so
+// that a workspace made for more items serves fewer too.
 template <class K, class P, class V>
 Layout layout(size_t n) {
   Layout l;
   if (n == 0) return l;
   constexpr size_t TILE = tile_items<K, P, V>();
   l.tiles = (n + TILE - 1) / TILE;
-  l.groups = (l.tiles + lookback::GROUP - 1) / lookback::GROUP;
-  // Descriptors, group words and the ticket: one span (lookback::state_layout).
-  const lookback::State st = lookback::state_layout(l.tiles);
-  l.desc = 0;
-  l.gagg = st.gagg * sizeof(uint64_t);
-  l.ginc = st.ginc * sizeof(uint64_t);
-  l.ticket = st.ticket * sizeof(uint64_t);
-  l.total = align_up(st.words * sizeof(uint64_t), 256);
+  l.total = align_up(lookback::state_words(l.tiles) * sizeof(uint64_t), 256);
   return l;
 }
 
@@ -328,9 +402,13 @@ rccl_hip_status run(const GroupArgs &a) {
   const Layout l = layout<K, P, V>(a.n);
   if (!a.ws || a.ws_bytes < l.total)
     return set_error(RCCL_HIP_ERROR_WORKSPACE_TOO_SMALL, "group workspace", l.total, a.ws_bytes);
-  unsigned char *ws = static_cast<unsigned char *>(a.ws);
-  uint64_t *desc = reinterpret_cast<uint64_t *>(ws + l.desc);
-  const size_t words = lookback::state_words(l.tiles);
+  uint64_t *desc = static_cast<uint64_t *>(a.ws);
+  const uint32_t subs = tiles_per_block(l.tiles);
+  const size_t blocks = (l.tiles + subs - 1) / subs;
+  // The state of `blocks` look-back tiles, in the place of the layout's, which
+  // has room for one per tile.
+  const lookback::State st = lookback::state_layout(blocks);
+  const size_t words = st.words;
   uint32_t nx = 1;
   RCCL_HIP_TRY(tile_order(&nx, a.stream));
   RCCL_HIP_TRY(fit_tile_order(reinterpret_cast<const void *>(&group_tile_kernel<K, P, Op, ITEMS>),
@@ -344,13 +422,12 @@ rccl_hip_status run(const GroupArgs &a) {
   {
     KernelTimer t("group_tile", a.stream, a.n);
     group_tile_kernel<K, P, Op, ITEMS>
-        <<<dim3(static_cast<uint32_t>(nx == XCDS ? xcd_order_grid(l.tiles, XCD_RUN) : l.tiles)),
+        <<<dim3(static_cast<uint32_t>(nx == XCDS ? xcd_order_grid(blocks, XCD_RUN) : blocks)),
            THREADS, 0, a.stream>>>(
-        static_cast<const K *>(a.keys), static_cast<const P *>(a.pays),
-        static_cast<const V *>(a.vals), a.n, l.tiles, static_cast<K *>(a.out_keys),
-        static_cast<P *>(a.out_pays), static_cast<V *>(a.out_vals), a.out_count, desc,
-        reinterpret_cast<uint64_t *>(ws + l.gagg), reinterpret_cast<uint64_t *>(ws + l.ginc),
-        reinterpret_cast<uint64_t *>(ws + l.ticket), nx);
+            static_cast<const K *>(a.keys), static_cast<const P *>(a.pays),
+            static_cast<const V *>(a.vals), a.n, blocks, static_cast<K *>(a.out_keys),
+            static_cast<P *>(a.out_pays), static_cast<V *>(a.out_vals), a.out_count, desc,
+            desc + st.gagg, desc + st.ginc, desc + st.ticket, nx, subs);
   }
   return check_launch("group tile");
 }

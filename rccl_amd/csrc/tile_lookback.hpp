@@ -31,20 +31,25 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
   return v;
 }
 
-// Called by the 64 lanes of one wave of tile t (of `tiles`), whose count is
-// tile_count. desc holds `tiles` words, gagg and ginc one word per group, all
-// zero before the launch. Returns the sum of the counts of tiles 0..t-1 (in
-// every lane).
-__device__ __forceinline__ uint64_t tile_prefix(size_t t, size_t tiles, uint64_t tile_count,
-                                                uint64_t *desc, uint64_t *gagg, uint64_t *ginc,
-                                                uint32_t lane) {
+// Publishes tile t's count (one lane). A kernel that has work left between its
+// count and its offset calls this first and tile_resolve after the work, so
+// that later tiles need not wait for it.
+__device__ __forceinline__ void tile_publish(size_t t, uint64_t tile_count, uint64_t *desc,
+                                             uint64_t *gagg) {
+  store_agent(&desc[t], (t == 0 ? F_INCL : F_AGG) | tile_count);
+  add_agent(&gagg[t / GROUP], uint64_t((1ull << GA_SHIFT) | tile_count));
+}
+
+// Called by the 64 lanes of one wave of tile t (of `tiles`), whose count,
+// tile_count, has been published. desc holds `tiles` words, gagg and ginc one
+// word per group, all zero before the launch. Returns the sum of the counts of
+// tiles 0..t-1 (in every lane).
+__device__ __forceinline__ uint64_t tile_resolve(size_t t, size_t tiles, uint64_t tile_count,
+                                                 uint64_t *desc, uint64_t *gagg, uint64_t *ginc,
+                                                 uint32_t lane) {
   const size_t g = t / GROUP;
   const size_t gfirst = g * GROUP;
   const uint32_t pos = static_cast<uint32_t>(t - gfirst);
-  if (lane == 0) {
-    store_agent(&desc[t], (t == 0 ? F_INCL : F_AGG) | tile_count);
-    add_agent(&gagg[g], uint64_t((1ull << GA_SHIFT) | tile_count));
-  }
   uint64_t prefix = 0;
   if (t > 0) {
     bool done = false;
@@ -108,6 +113,14 @@ __device__ __forceinline__ uint64_t tile_prefix(size_t t, size_t tiles, uint64_t
   const size_t glast = std::min(gfirst + GROUP, tiles) - 1;
   if (lane == 0 && t == glast) store_agent(&ginc[g], F_INCL | (prefix + tile_count));
   return prefix;
+}
+
+// Both in one: publish, then look back.
+__device__ __forceinline__ uint64_t tile_prefix(size_t t, size_t tiles, uint64_t tile_count,
+                                                uint64_t *desc, uint64_t *gagg, uint64_t *ginc,
+                                                uint32_t lane) {
+  if (lane == 0) tile_publish(t, tile_count, desc, gagg);
+  return tile_resolve(t, tiles, tile_count, desc, gagg, ginc, lane);
 }
 
 // Look-back state of `tiles` tiles, as word offsets into one span that is
