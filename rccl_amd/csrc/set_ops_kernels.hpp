@@ -531,11 +531,19 @@ tile_kernel(const K *__restrict__ a, const V *__restrict__ av, const K *__restri
   // Two-level decoupled look-back for the block's output offset (wave 0),
   // while the other waves compact the first sub-tile into LDS (every read of
   // the staged inputs lies before the last scan barrier).
+  // A counted operation needs the sum of the counts and no block's offset: no
+  // block waits (2 x 2^25 u64 keys: 204-220 us with the look-back, 169-202 here).
   if (wave == 0) {
-    const uint64_t prefix = lookback::tile_prefix(t, lb_tiles, total, desc, gagg, ginc, lane);
-    if (lane == 0) {
-      if (t + 1 == lb_tiles && out_count) *out_count = prefix + total;
-      sm.tile_offset = prefix;
+    if (out == nullptr && lb_tiles <= lookback::SUM_TILES) {
+      uint64_t sum = 0;
+      if (lane == 0 && lookback::tile_sum(t, lb_tiles, total, gagg, ginc, sum) && out_count)
+        *out_count = sum;
+    } else {
+      const uint64_t prefix = lookback::tile_prefix(t, lb_tiles, total, desc, gagg, ginc, lane);
+      if (lane == 0) {
+        if (t + 1 == lb_tiles && out_count) *out_count = prefix + total;
+        sm.tile_offset = prefix;
+      }
     }
   }
   if (out != nullptr) compact(sub[0]);

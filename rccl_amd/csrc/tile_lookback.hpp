@@ -123,6 +123,26 @@ __device__ __forceinline__ uint64_t tile_prefix(size_t t, size_t tiles, uint64_t
   return tile_resolve(t, tiles, tile_count, desc, gagg, ginc, lane);
 }
 
+// For a launch that wants only the sum of all counts: no tile waits for another.
+// The tile that completes its group's aggregate (gagg) adds it to `all`, and
+// the one that completes that has the sum: at most GROUP additions meet on a
+// group's word and one per group on `all`. Called by one lane; gagg and all are
+// zero before the launch, and tiles is at most SUM_TILES (the group count has
+// 16 bits). Returns whether this tile was the last, with the sum.
+constexpr size_t SUM_TILES = GROUP * 0xffff;
+__device__ __forceinline__ bool tile_sum(size_t t, size_t tiles, uint64_t tile_count,
+                                         uint64_t *gagg, uint64_t *all, uint64_t &sum) {
+  const size_t g = t / GROUP, groups = (tiles + GROUP - 1) / GROUP;
+  const uint64_t members = std::min(GROUP, tiles - g * GROUP);
+  const uint64_t group = add_agent(&gagg[g], uint64_t((1ull << GA_SHIFT) | tile_count));
+  if ((group >> GA_SHIFT) + 1 != members) return false;
+  const uint64_t part = (group & GA_MASK) + tile_count;
+  const uint64_t before = add_agent(all, uint64_t((1ull << GA_SHIFT) | part));
+  if ((before >> GA_SHIFT) + 1 != groups) return false;
+  sum = (before & GA_MASK) + part;
+  return true;
+}
+
 // Look-back state of `tiles` tiles, as word offsets into one span that is
 // zeroed before a launch: tile descriptors, a gap of GAP words, group
 // aggregates, another gap, group prefixes, the tile ticket. The gaps keep the
